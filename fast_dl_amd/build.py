@@ -43,7 +43,7 @@ DEVICE_FLAGS = [
 COMMON_FLAGS = ["-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-result",
                 "-I", INCLUDE, "-I", CSRC]
 
-GEMM_SOURCES = ["sgemm.hip", "mlp_kernels.hip", "data_kernels.hip", "capi.hip"]
+GEMM_SOURCES = ["sgemm.hip", "mlp_kernels.hip", "row_kernels.hip", "data_kernels.hip", "capi.hip"]
 DL_SOURCES_DIR = os.path.join(CSRC, "dl")
 
 

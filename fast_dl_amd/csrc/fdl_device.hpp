@@ -18,6 +18,36 @@ namespace fdl {
 // issued.  On the main path nothing is outstanding here, so this costs nothing.
 __device__ __forceinline__ void wait_vmem_idle() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
+// Lane exchanges within a half-wave (32 lanes) for row reductions.
+// Step 0 pairs lane i with i ^ 16 (ds_swizzle), step 1 with 15 - i within
+// 16 lanes (DPP row_mirror), step 2 with 7 - i within 8 (row_half_mirror),
+// steps 3 and 4 with i ^ 2 and i ^ 1 (quad permutations).  Step s always
+// pairs lanes that differ in bit 4 - s and agree in the bits above it, so
+// applying op(x, partner(x)) for s = 0..4 reduces over all 32 lanes and
+// leaves the same value on every lane (each pair computes a op b and b op a).
+template <int kCtrl>
+__device__ __forceinline__ float dpp_mov(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
+                                                                 kCtrl, 0xF, 0xF, false));
+}
+
+template <int kStep>
+__device__ __forceinline__ float half_wave_partner(float x) {
+    if constexpr (kStep == 0) {
+        constexpr int kXor16 = 0x401F;  // ds_swizzle bit mode: and 0x1f, xor 0x10
+        return __builtin_bit_cast(float,
+                                  __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, x), kXor16));
+    } else if constexpr (kStep == 1) {
+        return dpp_mov<0x140>(x);  // row_mirror
+    } else if constexpr (kStep == 2) {
+        return dpp_mov<0x141>(x);  // row_half_mirror
+    } else if constexpr (kStep == 3) {
+        return dpp_mov<0x4E>(x);   // quad_perm [2, 3, 0, 1]
+    } else {
+        return dpp_mov<0xB1>(x);   // quad_perm [1, 0, 3, 2]
+    }
+}
+
 // Column sums of a row-major rows x cols matrix, 32 columns per block and 8
 // row groups per column (256 threads).  Row groups are added in group order,
 // so the result is deterministic.  With `param`, the block also applies

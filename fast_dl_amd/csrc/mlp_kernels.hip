@@ -1,6 +1,6 @@
-// Elementwise and row kernels around the GEMM: bias, ReLU forward/backward,
-// column sums, row softmax, softmax cross-entropy (loss and gradient), SGD
-// and the Philox random fills.  All are HBM- or latency-bound; none uses
+// Kernels around the GEMM: bias, ReLU forward/backward, column sums, the MLP
+// step's head, SGD and the Philox random fills (row softmax and softmax
+// cross-entropy are in row_kernels.hip).  All are HBM- or latency-bound; none uses
 // atomics, so every result is deterministic run to run.
 #include "fdl_device.hpp"
 #include "fdl_internal.hpp"
@@ -75,71 +75,10 @@ colsum_kernel(const float* __restrict__ x, float* __restrict__ out,
     colsum_body(x, out, param, lr, rows, cols, blockIdx.x);
 }
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;
-}
-
-// Row softmax: one wave per row, 4 rows per block.
-__global__ void softmax_kernel(const float* __restrict__ in, float* __restrict__ out,
-                               int64_t rows, int64_t cols) {
-    const int lane = threadIdx.x & 63;
-    const int64_t row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const float* x = in + row * cols;
-    float* y = out + row * cols;
-    float mx = -INFINITY;
-    for (int64_t c = lane; c < cols; c += 64) mx = fmaxf(mx, x[c]);
-    mx = wave_max(mx);
-    float s = 0.0f;
-    for (int64_t c = lane; c < cols; c += 64) s += expf(x[c] - mx);
-    s = wave_sum(s);
-    for (int64_t c = lane; c < cols; c += 64) y[c] = expf(x[c] - mx) / s;
-}
-
-// Softmax cross-entropy over the whole batch in one block: thread t owns rows
-// t, t+256, ...; per-thread loss partials are combined by a fixed tree, so
-// the loss is deterministic (the reference used a float atomicAdd per row).
-__global__ void __launch_bounds__(kBlock)
-softmax_xent_kernel(const float* __restrict__ logits,
-                    const int64_t* __restrict__ labels, float* __restrict__ loss,
-                    float* __restrict__ grad, int64_t batch, int64_t classes) {
-    __shared__ float part[kBlock];
-    const float inv_b = 1.0f / (float)batch;
-    float lsum = 0.0f;
-    for (int64_t row = threadIdx.x; row < batch; row += kBlock) {
-        const float* z = logits + row * classes;
-        float mx = z[0];
-        for (int64_t c = 1; c < classes; ++c) mx = fmaxf(mx, z[c]);
-        float s = 0.0f;
-        for (int64_t c = 0; c < classes; ++c) s += expf(z[c] - mx);
-        const int64_t label = labels[row];
-        const bool valid = label >= 0 && label < classes;
-        if (valid) lsum += (logf(s) + mx - z[label]) * inv_b;
-        if (grad) {
-            float* g = grad + row * classes;
-            const float inv_s = 1.0f / s;
-            for (int64_t c = 0; c < classes; ++c) {
-                float pc = expf(z[c] - mx) * inv_s;
-                if (valid && c == label) pc -= 1.0f;
-                g[c] = pc * inv_b;
-            }
-        }
-    }
-    part[threadIdx.x] = lsum;
-    __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0 && loss) loss[0] = part[0];
 }
 
 // Softmax cross-entropy for classes <= kXentFusedMaxClasses with the bias
@@ -238,36 +177,6 @@ softmax_xent_db_sgd_kernel(const float* __restrict__ logits,
 // The block's record at part + block * (classes + 1): the column sums of its
 // G2 rows (rows in order), then the sum of its rows' loss shares;
 // xent_finalize_body adds the records in block order.
-// Lane exchanges within a half-wave (32 lanes) for the head's reductions.
-// Step 0 pairs lane i with i ^ 16 (ds_swizzle), step 1 with 15 - i within
-// 16 lanes (DPP row_mirror), step 2 with 7 - i within 8 (row_half_mirror),
-// steps 3 and 4 with i ^ 2 and i ^ 1 (quad permutations).  Step s always
-// pairs lanes that differ in bit 4 - s and agree in the bits above it, so
-// applying op(x, partner(x)) for s = 0..4 reduces over all 32 lanes and
-// leaves the same value on every lane (each pair computes a op b and b op a).
-template <int kCtrl>
-__device__ __forceinline__ float dpp_mov(float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
-                                                                 kCtrl, 0xF, 0xF, false));
-}
-
-template <int kStep>
-__device__ __forceinline__ float half_wave_partner(float x) {
-    if constexpr (kStep == 0) {
-        constexpr int kXor16 = 0x401F;  // ds_swizzle bit mode: and 0x1f, xor 0x10
-        return __builtin_bit_cast(float,
-                                  __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, x), kXor16));
-    } else if constexpr (kStep == 1) {
-        return dpp_mov<0x140>(x);  // row_mirror
-    } else if constexpr (kStep == 2) {
-        return dpp_mov<0x141>(x);  // row_half_mirror
-    } else if constexpr (kStep == 3) {
-        return dpp_mov<0x4E>(x);   // quad_perm [2, 3, 0, 1]
-    } else {
-        return dpp_mov<0xB1>(x);   // quad_perm [1, 0, 3, 2]
-    }
-}
-
 __device__ __forceinline__ float half_wave_max(float x) {
     x = fmaxf(x, half_wave_partner<0>(x));
     x = fmaxf(x, half_wave_partner<1>(x));
@@ -901,23 +810,6 @@ hipError_t launch_colsum_sgd(const float* x, float* out, float* param, float lr,
 hipError_t launch_colsum(const float* x, float* out, int64_t rows, int64_t cols,
                          hipStream_t stream) {
     return launch_colsum_sgd(x, out, nullptr, 0.0f, rows, cols, stream);
-}
-
-hipError_t launch_softmax(const float* in, float* out, int64_t rows, int64_t cols,
-                          hipStream_t stream) {
-    if (rows == 0 || cols == 0) return hipSuccess;
-    const unsigned blocks = (unsigned)((rows + 3) / 4);
-    hipLaunchKernelGGL(softmax_kernel, dim3(blocks), dim3(kBlock), 0, stream, in,
-                       out, rows, cols);
-    return hipGetLastError();
-}
-
-hipError_t launch_softmax_xent(const float* logits, const int64_t* labels,
-                               float* loss, float* grad, int64_t batch,
-                               int64_t classes, hipStream_t stream) {
-    hipLaunchKernelGGL(softmax_xent_kernel, dim3(1), dim3(kBlock), 0, stream,
-                       logits, labels, loss, grad, batch, classes);
-    return hipGetLastError();
 }
 
 hipError_t launch_softmax_xent_db_sgd(const float* logits, const int64_t* labels,

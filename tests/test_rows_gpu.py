@@ -1,0 +1,108 @@
+"""Row softmax and softmax cross-entropy at the edges of their row forms.
+
+A row of up to 2048 columns sits in the registers of 4, 16 or 64 lanes (with
+16-byte accesses where rows are 16-byte aligned and longer than 64 columns),
+longer rows take a block each; the cross-entropy runs on one block or, with a
+gradient buffer, on many with their loss sums kept in its first floats.
+References are numpy in fp64.  Bounds: an exponential is within 2 ulp, its
+argument's rounding adds eps * |z - max|, a sum of n terms n * eps at most.
+"""
+import numpy as np
+import pytest
+
+import fast_dl_amd.capi as capi
+from tests.conftest import rng
+from tests.gpu_helpers import dev, host, say, stream
+
+pytestmark = pytest.mark.gpu
+
+EPS = float(np.finfo(np.float32).eps)
+
+# (rows, columns): both sides of every row form, with one block and with many
+SHAPES = [(1, 1), (700, 1), (257, 4), (769, 4), (3, 5), (600, 16), (129, 17), (300, 64),
+          (33, 65), (20, 68), (40, 128), (41, 129), (5, 256), (35, 257), (64, 260), (37, 512),
+          (36, 513), (4, 1000), (2100, 1000), (50, 1023), (51, 1024), (34, 1025), (33, 1028),
+          (7, 2047), (70, 2048), (2, 2049), (40, 2049), (3, 7000), (4500, 10),
+          (17000, 66), (70000, 3)]
+
+
+def _softmax64(z):
+    z = z.astype(np.float64)
+    m = z.max(1, keepdims=True)
+    e = np.exp(z - m)
+    s = e.sum(1, keepdims=True)
+    spread = np.minimum(m - z, 200.0)  # beyond it the probability is below fp32's smallest
+    bound = (8.0 + spread + np.sum(e * spread, 1, keepdims=True) / s
+             + np.minimum(z.shape[1], 64)) * EPS
+    return e / s, np.log(s[:, 0]) + m[:, 0], bound
+
+
+def _offset(a, shift):
+    """A device copy of `a` that starts `shift` floats past an allocation."""
+    import torch
+
+    buf = torch.empty(a.size + shift, device="cuda")
+    view = buf[shift:].view(a.shape)
+    view.copy_(dev(a))
+    return view
+
+
+@pytest.mark.parametrize("rows,cols", SHAPES)
+@pytest.mark.parametrize("shift", [0, 1])
+def test_softmax_rows(device, rows, cols, shift):
+    import torch
+
+    z = (rng(rows * 3 + cols).standard_normal((rows, cols)) * 4).astype(np.float32)
+    if cols > 2:
+        z[::3, cols // 2] = -np.inf  # a masked column
+    d, out = _offset(z, shift), _offset(np.full_like(z, np.nan), shift)
+    say(f"softmax rows {rows}x{cols} shift={shift}")
+    capi.softmax(d.data_ptr(), out.data_ptr(), rows, cols, stream())
+    ref, _, bound = _softmax64(z)
+    assert np.all(np.abs(host(out) - ref) <= bound * ref + 1e-37)
+    capi.softmax(d.data_ptr(), d.data_ptr(), rows, cols, stream())  # in place
+    assert torch.equal(d, out)
+
+
+@pytest.mark.parametrize("batch,classes", SHAPES)
+@pytest.mark.parametrize("shift", [0, 1])
+def test_softmax_xent_rows(device, batch, classes, shift):
+    import torch
+
+    g = rng(batch * 7 + classes)
+    z = (g.standard_normal((batch, classes)) * 3).astype(np.float32)
+    lab = g.integers(0, classes, batch).astype(np.int64)
+    lab[::5] = [-1, classes, 1 << 40][batch % 3]  # no class: left out of the loss
+    d, dl = _offset(z, shift), dev(lab)
+    grad = _offset(np.full_like(z, np.nan), shift)
+    loss = torch.full((1,), float("nan"), device="cuda")
+    say(f"softmax_xent rows {batch}x{classes} shift={shift}")
+    capi.softmax_xent(d.data_ptr(), dl.data_ptr(), loss.data_ptr(), grad.data_ptr(), batch,
+                      classes, stream())
+    p, lse, bound = _softmax64(z)
+    valid = (lab >= 0) & (lab < classes)
+    at = np.flatnonzero(valid)
+    shares = np.zeros(batch)
+    shares[at] = lse[at] - z[at, lab[at]]
+    size = np.abs(lse) + np.abs(z).max(1) + 1.0
+    # each share rounds a few times, and passes through at most `adds` additions (a row
+    # group of one block takes every 16th row of wide ones)
+    adds = 160 + batch / 16
+    loss_tol = float(np.sum(size[at] * (bound.max(1)[at] + adds * EPS))) / batch + 1e-30
+    ref = p.copy()
+    ref[at, lab[at]] -= 1.0
+    grad_tol = (bound * p + 3 * EPS * np.abs(ref)) / batch + 1e-37
+    assert abs(float(host(loss)[0]) - shares.sum() / batch) <= loss_tol
+    assert np.all(np.abs(host(grad) - ref / batch) <= grad_tol)
+    # loss alone, gradient alone, and the gradient over the logits: the same rows
+    only = torch.full((1,), float("nan"), device="cuda")
+    capi.softmax_xent(d.data_ptr(), dl.data_ptr(), only.data_ptr(), None, batch, classes, stream())
+    assert abs(float(host(only)[0]) - shares.sum() / batch) <= loss_tol
+    alone = torch.full_like(grad, float("nan"))
+    capi.softmax_xent(d.data_ptr(), dl.data_ptr(), None, alone.data_ptr(), batch, classes,
+                      stream())
+    assert np.all(np.abs(host(alone) - ref / batch) <= grad_tol)
+    capi.softmax_xent(d.data_ptr(), dl.data_ptr(), only.data_ptr(), d.data_ptr(), batch, classes,
+                      stream())
+    assert abs(float(host(only)[0]) - shares.sum() / batch) <= loss_tol
+    assert np.all(np.abs(host(d) - ref / batch) <= grad_tol)
