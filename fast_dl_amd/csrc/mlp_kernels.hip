@@ -41,6 +41,82 @@ __device__ __forceinline__ void stage_to_lds(float* __restrict__ dst, const floa
     }
 }
 
+__device__ __forceinline__ float wave_sum(float v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+
+// Column sums of a tall matrix.  No block can add another's partial sums
+// without scratch memory, so each column is summed by one block and the
+// parallelism is across columns: strips of kTallCols columns (one 16-byte load
+// per row where rows are 16-byte aligned), 1024 threads of a block on 1024 rows at once, kUnroll rows
+// in flight each.  What bounds it is the cache lines a CU can take in, about
+// one per nanosecond whatever the width of the strip, so narrow strips on many
+// CUs win; the blocks whose strips share a 128-byte line are numbered onto one
+// XCD, whose L2 then fetches the line once (without that 60000 x 256 took 122
+// us, as eight fetches of everything).  60000 x 256: 154 -> 53 us, 60000 x 1024:
+// 242 -> 103 us, 4096 x 1024: 12.4 -> 8.0 us; wider strips (8, 16 and 32
+// columns) 99, 107 and 112 us at 60000 x 256.  Up to kColsumShort rows
+// colsum_kernel's one round trip is faster (1024 x 256: 2.9 against 3.1 us).
+constexpr int kTallThreads = 1024;
+constexpr int kTallCols = 4;
+constexpr int64_t kColsumShort = 2048;
+
+template <bool VEC>
+__global__ void __launch_bounds__(kTallThreads)
+colsum_tall_kernel(const float* __restrict__ x, float* __restrict__ out,
+                   float* __restrict__ param, float lr, int64_t rows, int64_t cols) {
+#pragma clang fp contract(off)
+    constexpr int V = kTallCols, kUnroll = 4;
+    constexpr int kWaves = kTallThreads / 64;
+    __shared__ float red[kWaves][V];
+    // strips in order over XCDs (block b runs on XCD b % 8), each a contiguous range
+    const int64_t per = gridDim.x / 8, extra = gridDim.x % 8;
+    const int64_t xcd = blockIdx.x % 8;
+    const int64_t c0 = (xcd * per + min(xcd, extra) + blockIdx.x / 8) * V;
+    const float* col = x + c0;
+    float s[V] = {};
+    for (int64_t r0 = threadIdx.x; r0 < rows; r0 += (int64_t)kUnroll * kTallThreads) {
+        float q[kUnroll][V];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            const float* p = col + min(r0 + u * (int64_t)kTallThreads, rows - 1) * cols;
+            if constexpr (VEC) {
+                const floatx4 z = *reinterpret_cast<const floatx4*>(p);
+#pragma unroll
+                for (int v = 0; v < V; ++v) q[u][v] = z[v];
+            } else {
+#pragma unroll
+                for (int v = 0; v < V; ++v) q[u][v] = p[min((int64_t)v, cols - 1 - c0)];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u)
+#pragma unroll
+            for (int v = 0; v < V; ++v)
+                s[v] += r0 + u * (int64_t)kTallThreads < rows ? q[u][v] : 0.0f;
+    }
+    // lanes by a fixed exchange tree, then the waves in order
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        s[v] = wave_sum(s[v]);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x / 64][v] = s[v];
+    }
+    __syncthreads();
+    const int64_t c = c0 + threadIdx.x;
+    if (threadIdx.x < V && c < cols) {
+        float t = red[0][threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) t += red[w][threadIdx.x];
+        out[c] = t;
+        if (param) {
+            const float step = lr * t;
+            param[c] -= step;
+        }
+    }
+}
+
 // out[r, c] += bias[c]   (src/kernels/cuda/bias.cu:5-12 semantics)
 __global__ void add_row_bias_kernel(float* __restrict__ out,
                                     const float* __restrict__ bias,
@@ -52,33 +128,90 @@ __global__ void add_row_bias_kernel(float* __restrict__ out,
     }
 }
 
-__global__ void relu_kernel(const float* __restrict__ in, float* __restrict__ out,
-                            int64_t n) {
-    for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < n;
-         idx += (int64_t)gridDim.x * blockDim.x) {
-        out[idx] = fmaxf(0.0f, in[idx]);
+// out[i] = op(a[i], b[i]) over n floats.  HBM-bound: 16 bytes per lane and
+// access where every operand is 16-byte aligned (`out` may be `a` or `b`), one
+// float per lane otherwise and for the last n % 4.  Outputs of kStreamBytes or
+// more leave through non-temporal stores, since no cache would hold them for
+// their reader.  15.4M floats: relu 36.8 -> 18.5 us (6.6 TB/s), relu_backward
+// 51.6 -> 32.1 us (5.7 TB/s); 65k floats 2.2 -> 2.0 us.  More than one access
+// per thread was no faster (2, 4 and 8: within 3%).
+struct OpRelu {
+    static constexpr bool kTwo = false;
+    float lr;
+    __device__ __forceinline__ float operator()(float a, float) const { return fmaxf(0.0f, a); }
+};
+struct OpReluBackward {
+    static constexpr bool kTwo = true;
+    float lr;
+    __device__ __forceinline__ float operator()(float g, float act) const {
+        return act > 0.0f ? g : 0.0f;
+    }
+};
+// The product is rounded before the subtraction (no FMA contraction), as the
+// reference's x86 host update computes it.
+struct OpSgd {
+    static constexpr bool kTwo = true;
+    float lr;
+    __device__ __forceinline__ float operator()(float p, float g) const {
+#pragma clang fp contract(off)
+        const float step = lr * g;
+        return p - step;
+    }
+};
+
+template <class Op, bool VEC, bool NT>
+__global__ void __launch_bounds__(kBlock)
+elementwise_kernel(const float* a, const float* b, float* out, int64_t n, Op op) {
+    const int64_t n4 = n / 4;
+    const int64_t units = VEC ? n4 + (n - 4 * n4) : n;
+    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < units;
+         i += (int64_t)gridDim.x * kBlock) {
+        if (VEC && i < n4) {
+            const floatx4 va = reinterpret_cast<const floatx4*>(a)[i];
+            floatx4 vb = va;
+            if constexpr (Op::kTwo) vb = reinterpret_cast<const floatx4*>(b)[i];
+            floatx4 r;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[e] = op(va[e], vb[e]);
+            floatx4* dst = reinterpret_cast<floatx4*>(out) + i;
+            if constexpr (NT) {
+                __builtin_nontemporal_store(r, dst);
+            } else {
+                *dst = r;
+            }
+        } else {
+            const int64_t e = VEC ? i + 3 * n4 : i;  // the last n % 4 floats follow the n4 units
+            out[e] = op(a[e], Op::kTwo ? b[e] : 0.0f);
+        }
     }
 }
 
-__global__ void relu_backward_kernel(const float* __restrict__ g,
-                                     const float* __restrict__ act,
-                                     float* __restrict__ out, int64_t n) {
-    for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < n;
-         idx += (int64_t)gridDim.x * blockDim.x) {
-        out[idx] = act[idx] > 0.0f ? g[idx] : 0.0f;
+constexpr int64_t kStreamBytes = int64_t(32) << 20;
+
+template <class Op>
+hipError_t launch_elementwise(const float* a, const float* b, float* out, int64_t n, Op op,
+                              bool streams, hipStream_t stream) {
+    if (n == 0) return hipSuccess;
+    const bool vec = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) |
+                       reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
+    const dim3 grid(grid_for(vec ? n / 4 + n % 4 : n));
+    if (!vec) {
+        hipLaunchKernelGGL((elementwise_kernel<Op, false, false>), grid, dim3(kBlock), 0, stream,
+                           a, b, out, n, op);
+    } else if (streams && n * (int64_t)sizeof(float) >= kStreamBytes) {
+        hipLaunchKernelGGL((elementwise_kernel<Op, true, true>), grid, dim3(kBlock), 0, stream, a,
+                           b, out, n, op);
+    } else {
+        hipLaunchKernelGGL((elementwise_kernel<Op, true, false>), grid, dim3(kBlock), 0, stream,
+                           a, b, out, n, op);
     }
+    return hipGetLastError();
 }
 
 __global__ void __launch_bounds__(kColsumThreads)
 colsum_kernel(const float* __restrict__ x, float* __restrict__ out,
               float* __restrict__ param, float lr, int64_t rows, int64_t cols) {
     colsum_body(x, out, param, lr, rows, cols, blockIdx.x);
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
 }
 
 // Softmax cross-entropy for classes <= kXentFusedMaxClasses with the bias
@@ -674,13 +807,6 @@ mlp_head_dx_kernel(int batch, int in_features, int hidden, int classes,
     }
 }
 
-// p -= lr * g with the product rounded before the subtraction (no FMA
-// contraction), as the reference's x86 host update computes it.
-__global__ void sgd_kernel(float* __restrict__ p, const float* __restrict__ g,
-                           float lr, int64_t n) {
-    sgd_body(p, g, lr, n, blockIdx.x, gridDim.x);
-}
-
 struct SgdMulti {
     float* p[4];
     const float* g[4];
@@ -784,23 +910,30 @@ hipError_t launch_add_row_bias(float* out, const float* bias, int64_t rows,
 }
 
 hipError_t launch_relu(const float* in, float* out, int64_t n, hipStream_t stream) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(relu_kernel, dim3(grid_for(n)), dim3(kBlock), 0, stream,
-                       in, out, n);
-    return hipGetLastError();
+    return launch_elementwise(in, nullptr, out, n, OpRelu{0.0f}, true, stream);
 }
 
 hipError_t launch_relu_backward(const float* g, const float* act, float* out,
                                 int64_t n, hipStream_t stream) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(relu_backward_kernel, dim3(grid_for(n)), dim3(kBlock), 0,
-                       stream, g, act, out, n);
-    return hipGetLastError();
+    return launch_elementwise(g, act, out, n, OpReluBackward{0.0f}, true, stream);
 }
 
 hipError_t launch_colsum_sgd(const float* x, float* out, float* param, float lr,
                              int64_t rows, int64_t cols, hipStream_t stream) {
     if (cols == 0) return hipSuccess;
+    // (a launch holds at most 2^32 threads: wider matrices keep the 32-column blocks)
+    if (rows > kColsumShort && cols <= (int64_t(1) << 23)) {
+        const bool vec = cols % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+        const dim3 grid((unsigned)((cols + kTallCols - 1) / kTallCols));
+        if (vec) {
+            hipLaunchKernelGGL((colsum_tall_kernel<true>), grid, dim3(kTallThreads), 0, stream, x,
+                               out, param, lr, rows, cols);
+        } else {
+            hipLaunchKernelGGL((colsum_tall_kernel<false>), grid, dim3(kTallThreads), 0, stream,
+                               x, out, param, lr, rows, cols);
+        }
+        return hipGetLastError();
+    }
     const unsigned blocks = (unsigned)((cols + kColsumCols - 1) / kColsumCols);
     hipLaunchKernelGGL(colsum_kernel, dim3(blocks), dim3(kColsumThreads), 0,
                        stream, x, out, param, lr, rows, cols);
@@ -871,12 +1004,10 @@ hipError_t launch_mlp_head_dx(const float* H, const float* W2, const float* b2,
     return hipGetLastError();
 }
 
+// (the parameter is read again by the next step's products: ordinary stores)
 hipError_t launch_sgd(float* param, const float* grad, float lr, int64_t n,
                       hipStream_t stream) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(sgd_kernel, dim3(grid_for(n, 4)), dim3(kBlock), 0, stream,
-                       param, grad, lr, n);
-    return hipGetLastError();
+    return launch_elementwise(param, grad, param, n, OpSgd{lr}, false, stream);
 }
 
 hipError_t launch_sgd_multi(int count, float* const* params,

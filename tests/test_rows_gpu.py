@@ -106,3 +106,42 @@ def test_softmax_xent_rows(device, batch, classes, shift):
                       stream())
     assert abs(float(host(only)[0]) - shares.sum() / batch) <= loss_tol
     assert np.all(np.abs(host(d) - ref / batch) <= grad_tol)
+
+
+@pytest.mark.parametrize("rows,cols", [(2049, 1), (2049, 3), (3000, 4), (2100, 34), (4096, 36),
+                                       (5119, 100), (9000, 257), (30001, 8)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_colsum_tall(device, rows, cols, shift):
+    import torch
+
+    x = rng(rows + cols).standard_normal((rows, cols)).astype(np.float32)
+    d = _offset(x, shift)
+    out = torch.full((cols + 1,), float("nan"), device="cuda")
+    say(f"colsum tall {rows}x{cols} shift={shift}")
+    capi.colsum(d.data_ptr(), out.data_ptr(), rows, cols, stream())
+    # a thread adds every 1024th row, then 6 exchanges and 16 waves
+    depth = rows / 1024 + 24
+    bound = depth * EPS * np.abs(x).astype(np.float64).sum(0)
+    assert np.all(np.abs(host(out)[:cols] - x.astype(np.float64).sum(0)) <= bound)
+    assert np.isnan(host(out)[cols])
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 1024, 1027, 65541, (8 << 20) + 5])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_elementwise(device, n, shift):
+    import torch
+
+    g = rng(n)
+    a, b = (g.standard_normal(n).astype(np.float32) for _ in range(2))
+    b[:: 7], b[:: 11] = 0.0, -0.0
+    a[:: 13] = np.nan
+    da, db = _offset(a, shift), _offset(b, shift)
+    out = _offset(np.zeros(n + 4, np.float32), shift)
+    say(f"elementwise n={n} shift={shift}")
+    capi.relu(da.data_ptr(), out.data_ptr(), n, stream())
+    assert np.array_equal(host(out)[:n], np.fmax(np.float32(0), a))
+    capi.relu_backward(da.data_ptr(), db.data_ptr(), out.data_ptr(), n, stream())
+    assert np.array_equal(host(out)[:n], np.where(b > 0, a, np.float32(0)), equal_nan=True)
+    capi.sgd_update(db.data_ptr(), da.data_ptr(), 0.3, n, stream())
+    assert np.array_equal(host(db), b - np.float32(0.3) * a, equal_nan=True)
+    assert torch.all(out[n:] == 0)
