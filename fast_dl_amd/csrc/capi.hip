@@ -125,6 +125,21 @@ int sgemm_impl(int transA, int transB, int64_t M, int64_t N, int64_t K, const fl
                      "sgemm launch failed");
 }
 
+fdl::GemmParams shape_params(int64_t M, int64_t N, int64_t K) {
+    fdl::GemmParams p{};
+    p.M = (int)M;
+    p.N = (int)N;
+    p.K = (int)K;
+    return p;
+}
+
+// Bytes of the skinny family's K split (0: the problem does not take it).
+size_t skinny_workspace(int transA, int transB, int64_t M, int64_t N, int64_t K, int64_t batch) {
+    if (!fits_int(M) || !fits_int(N) || !fits_int(K) || batch < 1) return 0;
+    return fdl::skinny_split_plan(shape_params(M, N, K), transA == FDL_OP_T, transB == FDL_OP_T,
+                                  batch).bytes;
+}
+
 // Scratch of fdl_sgemm_ex_noalloc: the partial sums of the skinny family's
 // K split (at most 4 MiB: M <= 8, N = K = 4096).  Each GPU holds its own copy
 // at its own address; host code reaches it only through the address
@@ -191,7 +206,9 @@ int fdl_sgemm_ex_noalloc(int transA, int transB, int64_t M, int64_t N, int64_t K
                          int64_t ldb, int64_t strideB, float* C, int64_t ldc,
                          int64_t strideC, int64_t batch, const float* bias,
                          const float* aux, int epilogue, void* stream) {
-    const size_t need = fdl_sgemm_workspace_size(transA, transB, M, N, K, batch);
+    // The skinny family's K split alone uses the shared scratch; products that
+    // could run as K slices take one launch here, as they need no exclusive use.
+    const size_t need = skinny_workspace(transA, transB, M, N, K, batch);
     if (need > kScratchBytes) {
         return fail(FDL_ERROR_INVALID_VALUE,
                     "sgemm_noalloc: the problem needs " + std::to_string(need) +
@@ -210,12 +227,10 @@ int fdl_sgemm_ex_noalloc(int transA, int transB, int64_t M, int64_t N, int64_t K
 
 size_t fdl_sgemm_workspace_size(int transA, int transB, int64_t M, int64_t N, int64_t K,
                                 int64_t batch) {
-    if (!fits_int(M) || !fits_int(N) || !fits_int(K) || batch < 1) return 0;
-    fdl::GemmParams p{};
-    p.M = (int)M;
-    p.N = (int)N;
-    p.K = (int)K;
-    return fdl::skinny_split_plan(p, transA == FDL_OP_T, transB == FDL_OP_T, batch).bytes;
+    const size_t skinny = skinny_workspace(transA, transB, M, N, K, batch);
+    if (skinny > 0 || !fits_int(M) || !fits_int(N) || !fits_int(K) || batch < 1) return skinny;
+    return fdl::slice_plan(shape_params(M, N, K), transA == FDL_OP_T, transB == FDL_OP_T, batch)
+        .bytes;
 }
 
 int fdl_sgemm_ex(int transA, int transB, int64_t M, int64_t N, int64_t K,
@@ -231,11 +246,8 @@ int fdl_sgemm_ex(int transA, int transB, int64_t M, int64_t N, int64_t K,
 int fdl_sgemm_kernel_choice(int transA, int transB, int64_t M, int64_t N, int64_t K,
                             int64_t batch) {
     if (!fits_int(M) || !fits_int(N) || !fits_int(K) || batch < 1) return FDL_KERNEL_AUTO;
-    fdl::GemmParams p{};
-    p.M = (int)M;
-    p.N = (int)N;
-    p.K = (int)K;
-    return static_cast<int>(fdl::choose_kernel(p, transA == FDL_OP_T, transB == FDL_OP_T, batch));
+    return static_cast<int>(fdl::choose_kernel(shape_params(M, N, K), transA == FDL_OP_T,
+                                               transB == FDL_OP_T, batch));
 }
 
 int fdl_gemm(const float* a, const float* b, float* c, int m, int n, int k) {

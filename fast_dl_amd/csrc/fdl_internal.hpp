@@ -31,6 +31,8 @@ struct GemmParams {
     const float* aux;   // same layout as C (ldc, strideC), or null
     float* upd;         // EPI_SGD: parameter updated in place, same layout as C
     float lr;           // EPI_SGD: learning rate
+    int kslice;         // K-slice launches: K is cut into slices of this many steps, one per
+                        // `batch` (the last one shorter), each to its own part of C
     int64_t lda, ldb, ldc;
     int64_t strideA, strideB, strideC;
     int M, N, K;
@@ -118,10 +120,21 @@ struct SkinnySplit {
 };
 SkinnySplit skinny_split_plan(const GemmParams& p, bool transA, bool transB, int64_t batch);
 
+// K-slice form of a product whose tiles leave most CUs idle (sgemm.hip):
+// `slices` products over kslice steps of K each, to `bytes` of workspace, then
+// a pass adding them.  slices == 0: the problem runs in one launch.
+struct SlicePlan {
+    int slices = 0, kslice = 0;
+    size_t bytes = 0;
+};
+SlicePlan slice_plan(const GemmParams& p, bool transA, bool transB, int64_t batch);
+
 // Launches `batch` problems (grid.y indexes the batch).  Returns a hipError_t.
 // With a workspace of at least skinny_split_plan(...).bytes, a problem the
 // skinny family runs takes the K-split form (when B is 16-byte
-// vectorisable); the workspace is written on `stream`.
+// vectorisable); with at least slice_plan(...).bytes, one that a split-K
+// kernel would run takes the K-slice form.  The workspace is written on
+// `stream`.
 hipError_t launch_sgemm(const GemmParams& p, bool transA, bool transB,
                         int64_t batch, GemmKernel kernel, hipStream_t stream,
                         float* workspace = nullptr, size_t workspace_bytes = 0);

@@ -574,9 +574,10 @@ sgemm_tiled_kernel(GemmParams p, int tiles_m, int tiles_n) {
 // ASM = 1: the steady-state K loop is a hand-scheduled one of dma_loops.inc
 // (CfgDma256W4 and CfgDma128W4, every layout; see its generator).
 template <int BM_, int BN_, int BK_, int WM_, int WN_, int STAGES_, int XPIPE_ = 0,
-          int ILV_ = 0, int KS_ = 1, int CW_ = 4, int WPE_ = 1, int ASM_ = 0>
+          int ILV_ = 0, int KS_ = 1, int CW_ = 4, int WPE_ = 1, int ASM_ = 0, int SLICED_ = 0>
 struct DmaCfg {
     static constexpr int ASM = ASM_;
+    static constexpr int SLICED = SLICED_;  // batches are slices of one problem's K
     static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_;
     static constexpr int STAGES = STAGES_;
     static constexpr int XPIPE = XPIPE_, ILV = ILV_, KS = KS_, CW = CW_;
@@ -956,6 +957,10 @@ sgemm_dma_kernel(const float* __restrict__ A0, const float* __restrict__ B0,
     const int n0 = tn * BN;
     const float* __restrict__ A = p.A + bz * p.strideA;
     const float* __restrict__ B = p.B + bz * p.strideB;
+    // (the host takes as many slices as hold a step of K, so none is empty)
+    if constexpr (Cfg::SLICED != 0) {
+        p.K = __builtin_amdgcn_readfirstlane(min(pa.kslice, K - (int)bz * pa.kslice));
+    }
 
     OpA opa;
     OpB opb;
@@ -1495,7 +1500,14 @@ sgemm_dma_kernel(const float* __restrict__ A0, const float* __restrict__ B0,
     // the four-stage short-K tile (CfgDma64S, K <= 128) writes as many bytes
     // of C as it reads (the C4 batch: 5.57 -> 5.25 us in the trace; for the
     // 64x64 and 96x32 tiles of 777^3 to 2048^3 they measured -1% to +2%).
-    constexpr int kStreamStores = ((BM >= 128 && BN >= 128) || S == 4) ? 1 : 0;
+    // A slice's sums are read again by the next launch, and lie in a workspace of
+    // whole tiles: every block stores without bounds tests.
+    constexpr int kStreamStores =
+        ((BM >= 128 && BN >= 128) || S == 4) && Cfg::SLICED == 0 ? 1 : 0;
+    if constexpr (Cfg::SLICED != 0) {
+        p.M = tiles_m * BM;
+        p.N = tiles_n * BN;
+    }
     store_wave_tile<FM, FN, kStreamStores>(acc, p, bz, m0 + wm0, n0 + wn0, half, l32, bias_pre);
 }
 
@@ -2396,6 +2408,50 @@ sgemm_skinny_sum_kernel(const float* __restrict__ part, int S, int N, GemmParams
     store_epilogue(v, p, p.C, p.aux, p.upd, (int64_t)m * p.ldc + j, j);
 }
 
+// The second launch of a product whose K is cut into slices (launch_sliced):
+// C = epi(sum of the S slices' partial products, in slice order).  A thread
+// takes 4 columns of one row; partial rows are `ldp` floats (whole tiles), so
+// its 16-byte loads stay inside the workspace.  `vec`: C's rows take 16-byte
+// stores.
+constexpr int kSumThreads = 256;
+__global__ void __launch_bounds__(kSumThreads)
+sgemm_slice_sum_kernel(const float* __restrict__ part, int S, int ldp, int64_t slice, int n4,
+                       int total, int vec, GemmParams p) {
+    constexpr int kBatch = 8;  // loads in flight
+    const int idx = blockIdx.x * kSumThreads + threadIdx.x;
+    if (idx >= total) return;
+    const int i = idx / n4;
+    const int j = 4 * (idx - i * n4);
+    const float* src = part + (int64_t)i * ldp + j;
+    floatx4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < S; s0 += kBatch) {
+        floatx4 x[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            x[u] = *reinterpret_cast<const floatx4*>(src + min(s0 + u, S - 1) * slice);
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            if (s0 + u < S) v += x[u];
+        }
+    }
+    const int64_t off = (int64_t)i * p.ldc + j;
+    const int e = p.epilogue;
+    if (vec && (e == EPI_NONE || e == EPI_BIAS || e == EPI_BIAS_RELU || e == EPI_RELU)) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (e == EPI_BIAS || e == EPI_BIAS_RELU) v[q] += p.bias[j + q];
+            if (e == EPI_RELU || e == EPI_BIAS_RELU) v[q] = fmaxf(0.0f, v[q]);
+        }
+        *reinterpret_cast<floatx4*>(p.C + off) = v;
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if (j + q < p.N) store_epilogue(v[q], p, p.C, p.aux, p.upd, off + q, j + q);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Host-side launchers.
 // ---------------------------------------------------------------------------
@@ -2502,6 +2558,34 @@ hipError_t launch_dma(const GemmParams& p, bool ta, bool tb, int nbatch, hipStre
         FDL_DMA_LAUNCH(true, true);
     }
 #undef FDL_DMA_LAUNCH
+    return hipGetLastError();
+}
+
+// C = epi(op(A) op(B)) as `slices` products over kslice steps of K each, every
+// one to its own tile-padded matrix in `ws`, and a second launch that adds
+// them in slice order.  For outputs whose tiles leave most CUs idle.
+template <class Cfg>
+hipError_t launch_sliced(const GemmParams& p, bool ta, bool tb, int slices, int kslice, float* ws,
+                         hipStream_t stream) {
+    static_assert(Cfg::SLICED != 0, "a K-slice configuration");
+    const int ldp = (p.N + Cfg::BN - 1) / Cfg::BN * Cfg::BN;
+    const int64_t slice = (int64_t)((p.M + Cfg::BM - 1) / Cfg::BM * Cfg::BM) * ldp;
+    GemmParams q = p;
+    q.strideA = ta ? kslice * p.lda : kslice;
+    q.strideB = tb ? kslice : kslice * p.ldb;
+    q.C = ws;
+    q.ldc = ldp;
+    q.strideC = slice;
+    q.kslice = kslice;
+    q.epilogue = EPI_NONE;
+    const hipError_t err = launch_dma<Cfg>(q, ta, tb, slices, stream);
+    if (err != hipSuccess) return err;
+    const int n4 = (p.N + 3) / 4;
+    const int total = p.M * n4;
+    const bool vec = p.N % 4 == 0 && p.ldc % 4 == 0 && aligned16(p.C);
+    hipLaunchKernelGGL(sgemm_slice_sum_kernel, dim3((total + kSumThreads - 1) / kSumThreads),
+                       dim3(kSumThreads), 0, stream, ws, slices, ldp, slice, n4, total, (int)vec,
+                       p);
     return hipGetLastError();
 }
 
@@ -2937,6 +3021,18 @@ using CfgDma64S = DmaCfg<64, 64, 16, 32, 32, 4, 0, 1>;
 // k-groups (777^3: 18.1 -> 17.4 us).
 using CfgDma96x32U = DmaCfg<96, 32, 64, 32, 32, 3, 1, 1, 4, 1>;
 using CfgDma128W8U = DmaCfg<128, 128, 64, 64, 32, 2, 1, 1, 1, 1>;
+// K-slice forms (launch_sliced): 64x64 tiles, and 32x64 ones for at most 32
+// rows, with 16- and with 4-byte copies.  Four k-group sets: one output sums a
+// quarter of its slice at a time, so the longest chain of additions is no
+// longer than in the split-K kernels, and neither is the error against fp64
+// (2.9e-7 of the norm at 512x512x4096 in four slices; with two sets 4.1e-7 at
+// 24.4 us against 24.4, with the hand-scheduled loop's one set 5.7e-7 at 23.6
+// us).  Two stages of the 64x64 tile leave room for two blocks per CU, where a
+// long K takes several rounds (eight slices there: 27.4 us against 29.8).
+using CfgSlice64 = DmaCfg<64, 64, 64, 32, 32, 2, 1, 1, 4, 4, 1, 0, 1>;
+using CfgSlice64U = DmaCfg<64, 64, 64, 32, 32, 2, 1, 1, 4, 1, 1, 0, 1>;
+using CfgSlice32 = DmaCfg<32, 64, 64, 32, 32, 3, 1, 1, 4, 4, 1, 0, 1>;
+using CfgSlice32U = DmaCfg<32, 64, 64, 32, 32, 3, 1, 1, 4, 1, 1, 0, 1>;
 
 // Dispatch cost model.  A config runs `slots` blocks per CU at full
 // occupancy (LDS and register bound), each block holding `waves` waves; eff[w]
@@ -3062,6 +3158,25 @@ const char* kernel_name(GemmKernel k) {
     return "unknown";
 }
 
+namespace {
+
+// Time of the split-K kernel with `tile`-wide tiles, in us: the blocks run in
+// rounds of one per CU, each bound by its own serial K (the lines of A and B a
+// CU takes in).  Measured (us, 16 / 32 wide): 128x1024x1024 7.3 / 11.0,
+// 2048x100x1024 13.4 / 11.4, 1024x100x2048 13.7 / 19.7, 32x4096x4096
+// 26.7 / 35.9, 64x64x4096 11.6 / 34.6, 512^3 7.9 / 6.9, 700^3 19.0 / 16.2;
+// B k-contiguous (NT): 256x784x256 5.6 / 4.5, 2048x100x1024 15.8 / 10.3.
+double splitk_us(int tile, const GemmParams& p, bool transB, int64_t batch) {
+    constexpr int64_t kCUs = 256;
+    const int64_t tiles =
+        (int64_t)((p.M + tile - 1) / tile) * ((p.N + tile - 1) / tile) * batch;
+    const double rounds = (double)((tiles + kCUs - 1) / kCUs);
+    return tile == 16 ? 1.5 + (transB ? 0.0037 : 0.0029) * p.K * rounds
+                      : 2.0 + 0.0087 * p.K * rounds;
+}
+
+}  // namespace
+
 GemmKernel choose_kernel(const GemmParams& p, bool transA, bool transB,
                          int64_t batch) {
     // Skinny M: one streaming pass over B on the VALU beats an MFMA tile
@@ -3070,8 +3185,8 @@ GemmKernel choose_kernel(const GemmParams& p, bool transA, bool transB,
     const int64_t t64 = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * batch;
     constexpr int64_t kCUs = 256;
     // Too few 64x64 tiles to occupy the GPU: split K over the waves of a
-    // block instead, with 16x16 output tiles when 32x32 ones would leave most
-    // CUs idle.  With K >= 256 the 64x64 direct-to-LDS tile wins from ~160
+    // block instead, on 16x16 or 32x32 output tiles by splitk_us (short K: 16x16
+    // when 32x32 ones would leave most CUs idle).  With K >= 256 the 64x64 direct-to-LDS tile wins from ~160
     // tiles (777^3: 21.9 vs 25.2 us; 1024^3: 22 vs 42 us).  Short K (64 to
     // 255) needs a full GPU of 64x64 tiles (the C4 batch of 64 128x128x64
     // problems: 5.0-5.2 vs 6.1-6.2 us for split-K; 1024x1024x128: 6.5 vs 8.4
@@ -3085,7 +3200,10 @@ GemmKernel choose_kernel(const GemmParams& p, bool transA, bool transB,
     if (p.K < 64 || t64 < (long_k ? 160 : kCUs) ||
         (!long_k && t128 < 128 && rem > 0 && rem < 64)) {
         const int64_t t32 = (int64_t)((p.M + 31) / 32) * ((p.N + 31) / 32) * batch;
-        return t32 < 128 ? GemmKernel::SplitK16 : GemmKernel::SplitK32;
+        if (p.K < 128) return t32 < 128 ? GemmKernel::SplitK16 : GemmKernel::SplitK32;
+        return splitk_us(16, p, transB, batch) < splitk_us(32, p, transB, batch)
+                   ? GemmKernel::SplitK16
+                   : GemmKernel::SplitK32;
     }
     // The direct-to-LDS tiles compete where their shape contract holds (the
     // 4-byte-copy ones almost always); the register-staged tiles only when
@@ -3167,7 +3285,79 @@ SkinnySplit skinny_split_plan(const GemmParams& p, bool transA, bool transB, int
     return s;
 }
 
+// When and how a product runs as K slices.  Only where a split-K kernel would
+// run it (its tiles cannot fill the GPU): the slices' tiles in r rounds of one
+// per CU take about 8.4 us (two launches, the first tile's arrival, the sums'
+// round trip) plus 0.0150 us per step of K (64x64 tile; 0.0082 for 32x64), 2
+// us per further round and the partial sums' bytes.  Measured against the
+// split-K kernel (us): 32x4096x4096 17.5 / 26.4, 64x4096x4096 23.8 / 36.8,
+// 512x512x4096 24.4 / 36.7, 300x300x3000 14.0 / 21.1, 776x500x2000 23.9 /
+// 37.3, 784x256x60000 TN 214 / 515, odd 32x4097x4099 22.3 / 73.4 and
+// 777x250x5000 TN 28 / 47.6; where it predicts less than a tenth to gain the
+// single launch stays (256x256x1024 9 / 4.4, 16x4096x4096 17.8 / 16.7).  From
+// the shape alone, since the workspace query has no leading dimensions or
+// pointers: these choose between 16- and 4-byte copies of the same tile.
+SlicePlan slice_plan(const GemmParams& p, bool transA, bool transB, int64_t batch) {
+    SlicePlan s;
+    if (batch != 1 || p.M < 1 || p.N < 1 || p.K < 256) return s;
+    const GemmKernel direct = choose_kernel(p, transA, transB, batch);
+    if (direct != GemmKernel::SplitK16 && direct != GemmKernel::SplitK32) return s;
+    // (operands that cannot take 16-byte loads cost the split-K kernels about a
+    // fifth more than splitk_us says: 16x1001x4097 18.2 us, 32x3001x2003 15.7)
+    const bool odd = p.K % 4 != 0 || (transA ? p.M : p.K) % 4 != 0 ||
+                     (transB ? p.K : p.N) % 4 != 0;
+    const double direct_us = (odd ? 1.2 : 1.0) *
+        splitk_us(direct == GemmKernel::SplitK16 ? 16 : 32, p, transB, batch);
+    const int bm = p.M <= 32 ? 32 : 64, bn = 64;
+    const int64_t tiles_m = (p.M + bm - 1) / bm, tiles_n = (p.N + bn - 1) / bn;
+    const int64_t tiles = tiles_m * tiles_n;
+    const double matrix = (double)tiles * bm * bn * sizeof(float);
+    const double per_step = bm == 32 ? 0.0082 : 0.0150;
+    constexpr int64_t kCUs = 256;
+    constexpr int kStep = 64;  // slices are whole K-tiles
+    constexpr double kMaxBytes = 32 << 20;
+    double best_us = 0.9 * direct_us;
+    for (int rounds = 1; rounds <= 6; ++rounds) {
+        int64_t slices = rounds * kCUs / tiles;
+        if (slices < 2) continue;
+        slices = std::min<int64_t>(slices, (int64_t)(kMaxBytes / matrix));
+        if (slices < 2) break;
+        const int64_t steps =
+            std::max<int64_t>(2 * kStep, ((p.K + slices - 1) / slices + kStep - 1) / kStep * kStep);
+        slices = (p.K + steps - 1) / steps;
+        if (slices < 2) break;
+        const int64_t run = (slices * tiles + kCUs - 1) / kCUs;
+        const double us = 8.4 + per_step * steps * run + 2.0 * (run - 1) +
+                          slices * matrix * 2.0 / 5.0e6;
+        if (us < best_us) {
+            best_us = us;
+            s.slices = (int)slices;
+            s.kslice = (int)steps;
+            s.bytes = (size_t)slices * tiles * bm * bn * sizeof(float);
+        }
+    }
+    return s;
+}
+
 namespace {
+
+// The K-slice launch of a plan, or hipErrorInvalidValue (nothing launched) for
+// operands none of its forms takes: a leading dimension past the copies' 32-bit
+// offsets, or misaligned beyond 4 bytes.
+hipError_t launch_slice_plan(const GemmParams& p, bool ta, bool tb, const SlicePlan& s, float* ws,
+                             hipStream_t stream) {
+    const int64_t sa = ta ? s.kslice * p.lda : s.kslice;
+    const int64_t sb = tb ? s.kslice : s.kslice * p.ldb;
+    if (sa > INT32_MAX || sb > INT32_MAX) return hipErrorInvalidValue;
+    const bool small = p.M <= 32;
+    if (dma_supported(GemmKernel::Dma64, p, ta, tb, 1)) {
+        return small ? launch_sliced<CfgSlice32>(p, ta, tb, s.slices, s.kslice, ws, stream)
+                     : launch_sliced<CfgSlice64>(p, ta, tb, s.slices, s.kslice, ws, stream);
+    }
+    if (!dma_supported(GemmKernel::Dma64U, p, ta, tb, 1)) return hipErrorInvalidValue;
+    return small ? launch_sliced<CfgSlice32U>(p, ta, tb, s.slices, s.kslice, ws, stream)
+                 : launch_sliced<CfgSlice64U>(p, ta, tb, s.slices, s.kslice, ws, stream);
+}
 
 GroupDev group_dev(const GroupJob& j) {
     GroupDev d{};
@@ -3318,6 +3508,15 @@ hipError_t launch_sgemm(const GemmParams& p0, bool transA, bool transB,
                      : kernel == GemmKernel::Dma128W8 ? GemmKernel::Tiled128W8
                      : kernel == GemmKernel::Dma128W8U ? GemmKernel::Tiled128W8
                                                       : GemmKernel::Tiled64;
+        }
+    }
+
+    if (automatic && workspace != nullptr &&
+        (kernel == GemmKernel::SplitK16 || kernel == GemmKernel::SplitK32)) {
+        const SlicePlan s = slice_plan(p0, transA, transB, batch);
+        if (s.slices > 0 && workspace_bytes >= s.bytes) {
+            const hipError_t err = launch_slice_plan(p0, transA, transB, s, workspace, stream);
+            if (err != hipErrorInvalidValue) return err;
         }
     }
 

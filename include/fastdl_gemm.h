@@ -139,11 +139,12 @@ int fdl_sgemm_kernel_choice(int transA, int transB,
 
 /*
  * Workspace, in bytes, that fdl_sgemm_ex_ws can use for this problem; 0 when
- * it would use none.  Non-zero only for one problem (batch == 1) that the
- * skinny family runs (M <= 8, transB == N) with N % 4 == 0 and enough work
- * to pay for a second pass (K >= 4096, or N * K >= 2^23).  This build's own extension: the
- * reference called cublasSgemm, which takes no workspace
- * (src/kernels/cuda/gemm.cu:166-177).
+ * it would use none.  Non-zero only for one problem (batch == 1) that pays
+ * for a second pass over partial sums: one the skinny family runs (M <= 8,
+ * transB == N) with N % 4 == 0 and K >= 4096 or N * K >= 2^23, or one with
+ * too few output tiles to fill the GPU and a long K (at most 32 MiB).  This
+ * build's own extension: the reference called cublasSgemm, which takes no
+ * workspace (src/kernels/cuda/gemm.cu:166-177).
  */
 size_t fdl_sgemm_workspace_size(int transA, int transB,
                                 int64_t M, int64_t N, int64_t K, int64_t batch);
@@ -154,8 +155,11 @@ size_t fdl_sgemm_workspace_size(int transA, int transB,
  * vectorisable, a skinny problem splits K over blocks: each block streams a
  * 256-column band of B over one slice of K and writes partial sums to the
  * workspace, and a second launch adds the slices in slice order and applies
- * the epilogue.  Results repeat bit for bit, and differ from fdl_sgemm_ex's
- * single pass only in the order of the fp32 additions.  Every other problem,
+ * the epilogue.  A product of few output tiles and a long K (a weight gradient
+ * over a large batch, a layer on a few dozen rows) likewise runs as slices of
+ * K on tiles, then the sum.  Results repeat bit for bit, and differ from
+ * fdl_sgemm_ex's single pass only in the order of the fp32 additions.  Every
+ * other problem,
  * or a smaller workspace, runs exactly as fdl_sgemm_ex.  The workspace is
  * written on `stream`: work on other streams must not use it until the call's
  * work there has finished.
@@ -176,12 +180,13 @@ int fdl_sgemm_ex_ws(int transA, int transB,
  * library call), for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid allocation).  It has no
  * counterpart in the reference.  The scratch is a static device array of
- * 4 MiB per GPU, held until the process ends; a problem whose
- * fdl_sgemm_workspace_size exceeds it returns FDL_ERROR_INVALID_VALUE.
- * Every call on one GPU shares that GPU's scratch: calls whose work overlaps
+ * 4 MiB per GPU, held until the process ends; only the skinny family's split
+ * uses it (every other problem runs as fdl_sgemm_ex), and one that needs more
+ * returns FDL_ERROR_INVALID_VALUE.
+ * Such calls on one GPU share that GPU's scratch: calls whose work overlaps
  * on one GPU (on different streams, or from different threads without
  * ordering between their streams) race and may return wrong results.
- * Results equal fdl_sgemm_ex_ws's bit for bit.
+ * A skinny problem's results equal fdl_sgemm_ex_ws's bit for bit.
  */
 int fdl_sgemm_ex_noalloc(int transA, int transB,
                          int64_t M, int64_t N, int64_t K,
