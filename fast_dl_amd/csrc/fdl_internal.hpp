@@ -129,6 +129,12 @@ struct SlicePlan {
 };
 SlicePlan slice_plan(const GemmParams& p, bool transA, bool transB, int64_t batch);
 
+// A weight gradient C = op(A) op(B) (EPI_NONE) of a large training step, over
+// as many slices of K as keep two blocks on every CU, in `scratch`
+// (16-byte aligned, or null); one launch where the scratch is too small.
+hipError_t launch_weight_grad(const GemmParams& p, bool transA, bool transB, float* scratch,
+                              size_t scratch_bytes, hipStream_t stream);
+
 // Launches `batch` problems (grid.y indexes the batch).  Returns a hipError_t.
 // With a workspace of at least skinny_split_plan(...).bytes, a problem the
 // skinny family runs takes the K-split form (when B is 16-byte
@@ -162,6 +168,11 @@ hipError_t launch_softmax(const float* in, float* out, int64_t rows,
 hipError_t launch_softmax_xent(const float* logits, const int64_t* labels,
                                float* loss, float* grad, int64_t batch,
                                int64_t classes, hipStream_t stream);
+// The gradient of launch_softmax_xent, its loss left as the sum of
+// xent_parts(batch, classes) partial sums at `part`.
+int64_t xent_parts(int64_t batch, int64_t classes);
+hipError_t launch_xent_parts(const float* logits, const int64_t* labels, float* part, float* grad,
+                             int64_t batch, int64_t classes, hipStream_t stream);
 // As launch_softmax_xent, and also db = column sums of the gradient and
 // bparam -= lr * db (the bias step of the layer that produced the logits).
 // Needs grad, db and bparam; classes <= kXentFusedMaxClasses.
@@ -212,6 +223,11 @@ hipError_t launch_sgd(float* param, const float* grad, float lr, int64_t n,
 hipError_t launch_sgd_multi(int count, float* const* params,
                             const float* const* grads, const int64_t* sizes,
                             float lr, hipStream_t stream);
+// db1 = column sums of G1 (rows x hidden), db2 = column sums of G2 (rows x
+// classes), loss = the sum of nparts floats `stride` apart from part.
+hipError_t launch_step_reduce(const float* G1, float* db1, int64_t hidden, const float* G2,
+                              float* db2, int64_t classes, int64_t rows, const float* part,
+                              int64_t nparts, int stride, float* loss, hipStream_t stream);
 // data[0 .. bytes) = 0 by a kernel (capturable, unlike a memset node).
 hipError_t launch_zero_fill(void* data, int64_t bytes, hipStream_t stream);
 hipError_t launch_fill_uniform(float* data, int64_t n, float low, float high,

@@ -263,14 +263,13 @@ struct TileLoader {
 // accumulators, whose top-left element is C[mw][nw], goes through the
 // epilogue into C.
 //
-// Interior wave blocks with an epilogue that reads nothing per element (none,
-// bias, bias+ReLU, ReLU) take a fast path: stores through a buffer descriptor
-// based at the block's corner, each lane's column and half-row as a 32-bit
-// offset and the row part wave-uniform (a scalar offset), so a store costs no
-// address arithmetic, no bounds test and no wait.  `bias_pre`, when given,
+// Stores go through a buffer descriptor based at the wave's corner, each lane's
+// column and half-row as a 32-bit offset and the row part wave-uniform (a
+// scalar offset), so a store costs no address arithmetic and no wait; blocks
+// on C's edge test each element's row and column.  `bias_pre`, when given,
 // holds this lane's bias value of each column block, fetched before the K
-// loop.  The per-element path below it serves edge blocks and the epilogues
-// that read aux or update a parameter.
+// loop.  The per-element path below it serves the epilogue that updates a
+// parameter and rows too long for 32-bit offsets.
 constexpr int kBufferWord3Store = 0x00020000;  // raw-buffer descriptor word 3 (gfx9 family)
 
 // STREAM = 1: the fast path's stores are non-temporal (buffer store `nt`), for
@@ -280,55 +279,112 @@ template <int FM, int FN, int STREAM = 0>
 __device__ __forceinline__ void store_wave_tile(floatx16 (&acc)[FM][FN], const GemmParams& p,
                                                 int64_t bz, int mw, int nw, int half,
                                                 int l32, const float* bias_pre = nullptr) {
-    {
+    // Byte offsets stay below 2^31: (FM * 32 rows) * ldc * 4 bytes.
+    if (p.epilogue != EPI_SGD && p.ldc < (int64_t(1) << 29) / (FM * 32)) {
         const int epi = p.epilogue;
-        const bool plain = epi == EPI_NONE || epi == EPI_BIAS || epi == EPI_BIAS_RELU ||
-                           epi == EPI_RELU;
-        // Byte offsets stay below 2^31: (FM * 32 rows) * ldc * 4 bytes.
-        if (plain && mw + FM * 32 <= p.M && nw + FN * 32 <= p.N &&
-            p.ldc < (int64_t(1) << 29) / (FM * 32)) {
-            const bool has_bias = epi == EPI_BIAS || epi == EPI_BIAS_RELU;
-            const bool relu = epi == EPI_BIAS_RELU || epi == EPI_RELU;
-            // mw and nw are wave-uniform by construction; saying so keeps the
-            // descriptor in scalar registers.
-            const int mwu = __builtin_amdgcn_readfirstlane(mw);
-            const int nwu = __builtin_amdgcn_readfirstlane(nw);
-            float* corner = p.C + bz * p.strideC + (int64_t)mwu * p.ldc + nwu;
-            const __amdgpu_buffer_rsrc_t rsrc =
-                __builtin_amdgcn_make_buffer_rsrc(corner, (short)0, -1, kBufferWord3Store);
-            const int ldc = (int)p.ldc;
-            const uint32_t lane_off = (uint32_t)((4 * half) * ldc + l32) * 4u;
-            float bj[FN];
-#pragma unroll
-            for (int ni = 0; ni < FN; ++ni) {
-                bj[ni] = has_bias ? (bias_pre ? bias_pre[ni] : p.bias[nw + ni * 32 + l32]) : 0.0f;
+        const bool has_bias = epi == EPI_BIAS || epi == EPI_BIAS_RELU;
+        const bool relu = epi == EPI_BIAS_RELU || epi == EPI_RELU;
+        // mw and nw are wave-uniform by construction; saying so keeps the
+        // descriptors in scalar registers.
+        const int mwu = __builtin_amdgcn_readfirstlane(mw);
+        const int nwu = __builtin_amdgcn_readfirstlane(nw);
+        const int rows = p.M - mwu;  // (edge blocks: rows and columns inside C)
+        const int cols = p.N - nwu;
+        if (rows <= 0 || cols <= 0) return;
+        const bool inside = rows >= FM * 32 && cols >= FN * 32;
+        const int64_t corner = bz * p.strideC + (int64_t)mwu * p.ldc + nwu;
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            p.C + corner, (short)0, -1, kBufferWord3Store);
+        const int ldc = (int)p.ldc;
+        const uint32_t lane_off = (uint32_t)((4 * half) * ldc + l32) * 4u;
+        // Element r of block (mi, ni) is row mi * 32 + 8 (r / 4) + r % 4 + 4 half,
+        // column ni * 32 + l32 of the wave's tile.
+        auto put = [&](auto edge, int mi, int ni, int r, float v) __attribute__((always_inline)) {
+            const int row = mi * 32 + 8 * (r >> 2) + (r & 3);
+            if (!decltype(edge)::value || (row + 4 * half < rows && ni * 32 + l32 < cols)) {
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc,
+                                                      (int)lane_off, (row * ldc + ni * 32) * 4,
+                                                      STREAM ? 2 : 0);  // 2: nt
             }
-            // One uniform branch on the epilogue, then straight-line stores.
-            auto store_all = [&](auto op) __attribute__((always_inline)) {
+        };
+        using Edge = std::true_type;
+        using Inside = std::false_type;
+        if (epi == EPI_RELU_GRAD) {
+            // The ReLU-backward mask: each 32x32 block's 16 mask values loaded
+            // together ahead of its stores, two blocks at a time (one by one, each
+            // load waits out the stores before it).  2048x1024x100 14.2 -> 9.4 us,
+            // 4096x4096x256 200 -> 87 us.
+            const __amdgpu_buffer_rsrc_t raux = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float*>(p.aux) + corner, (short)0, -1, kBufferWord3Store);
+            constexpr int kBlocks = FM * FN;
+            constexpr int kPair = kBlocks > 1 ? 2 : 1;
+            auto masked = [&](auto edge) __attribute__((always_inline)) {
 #pragma unroll
-                for (int ni = 0; ni < FN; ++ni)
+                for (int b0 = 0; b0 < kBlocks; b0 += kPair) {
+                    float mask[kPair][16];
 #pragma unroll
-                    for (int mi = 0; mi < FM; ++mi)
+                    for (int b = 0; b < kPair; ++b)
 #pragma unroll
                         for (int r = 0; r < 16; ++r) {
+                            const int mi = (b0 + b) % FM, ni = (b0 + b) / FM;
                             const int row = mi * 32 + 8 * (r >> 2) + (r & 3);
-                            const float v = op(acc[mi][ni][r], bj[ni]);
-                            __builtin_amdgcn_raw_buffer_store_b32(
-                                __builtin_bit_cast(uint32_t, v), rsrc, (int)lane_off,
-                                (row * ldc + ni * 32) * 4, STREAM ? 2 : 0);  // 2: nt
+                            int off = (int)lane_off, base = (row * ldc + ni * 32) * 4;
+                            if constexpr (decltype(edge)::value) {  // clamped into C
+                                off = (min(row + 4 * half, rows - 1) * ldc +
+                                       min(ni * 32 + l32, cols - 1)) * 4;
+                                base = 0;
+                            }
+                            mask[b][r] = __builtin_bit_cast(
+                                float, __builtin_amdgcn_raw_buffer_load_b32(raux, off, base, 0));
                         }
+#pragma unroll
+                    for (int b = 0; b < kPair; ++b)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            const int mi = (b0 + b) % FM, ni = (b0 + b) / FM;
+                            put(edge, mi, ni, r, mask[b][r] > 0.0f ? acc[mi][ni][r] : 0.0f);
+                        }
+                }
             };
-            if (has_bias && relu) {
-                store_all([](float v, float b) { return fmaxf(0.0f, v + b); });
-            } else if (has_bias) {
-                store_all([](float v, float b) { return v + b; });
-            } else if (relu) {
-                store_all([](float v, float) { return fmaxf(0.0f, v); });
+            if (inside) {
+                masked(Inside{});
             } else {
-                store_all([](float v, float) { return v; });
+                masked(Edge{});
             }
             return;
         }
+        float bj[FN];
+#pragma unroll
+        for (int ni = 0; ni < FN; ++ni) {
+            bj[ni] = !has_bias ? 0.0f
+                     : bias_pre ? bias_pre[ni]
+                                : p.bias[min(nw + ni * 32 + l32, p.N - 1)];
+        }
+        // One uniform branch on the epilogue, then straight-line stores.
+        auto store_all = [&](auto edge, auto op) __attribute__((always_inline)) {
+#pragma unroll
+            for (int ni = 0; ni < FN; ++ni)
+#pragma unroll
+                for (int mi = 0; mi < FM; ++mi)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) put(edge, mi, ni, r, op(acc[mi][ni][r], bj[ni]));
+        };
+        if (!inside) {
+            // (one copy of the code: the epilogue by selects)
+            store_all(Edge{}, [&](float v, float b) {
+                v = has_bias ? v + b : v;
+                return relu ? fmaxf(0.0f, v) : v;
+            });
+        } else if (has_bias && relu) {
+            store_all(Inside{}, [](float v, float b) { return fmaxf(0.0f, v + b); });
+        } else if (has_bias) {
+            store_all(Inside{}, [](float v, float b) { return v + b; });
+        } else if (relu) {
+            store_all(Inside{}, [](float v, float) { return fmaxf(0.0f, v); });
+        } else {
+            store_all(Inside{}, [](float v, float) { return v; });
+        }
+        return;
     }
     float* __restrict__ C = p.C + bz * p.strideC;
     const float* __restrict__ aux = p.aux ? p.aux + bz * p.strideC : nullptr;
@@ -1500,14 +1556,9 @@ sgemm_dma_kernel(const float* __restrict__ A0, const float* __restrict__ B0,
     // the four-stage short-K tile (CfgDma64S, K <= 128) writes as many bytes
     // of C as it reads (the C4 batch: 5.57 -> 5.25 us in the trace; for the
     // 64x64 and 96x32 tiles of 777^3 to 2048^3 they measured -1% to +2%).
-    // A slice's sums are read again by the next launch, and lie in a workspace of
-    // whole tiles: every block stores without bounds tests.
+    // (A slice's sums are read again by the next launch.)
     constexpr int kStreamStores =
         ((BM >= 128 && BN >= 128) || S == 4) && Cfg::SLICED == 0 ? 1 : 0;
-    if constexpr (Cfg::SLICED != 0) {
-        p.M = tiles_m * BM;
-        p.N = tiles_n * BN;
-    }
     store_wave_tile<FM, FN, kStreamStores>(acc, p, bz, m0 + wm0, n0 + wn0, half, l32, bias_pre);
 }
 
@@ -2410,8 +2461,8 @@ sgemm_skinny_sum_kernel(const float* __restrict__ part, int S, int N, GemmParams
 
 // The second launch of a product whose K is cut into slices (launch_sliced):
 // C = epi(sum of the S slices' partial products, in slice order).  A thread
-// takes 4 columns of one row; partial rows are `ldp` floats (whole tiles), so
-// its 16-byte loads stay inside the workspace.  `vec`: C's rows take 16-byte
+// takes 4 columns of one row; partial rows are `ldp` floats (N rounded up to a
+// multiple of 4), so its 16-byte loads stay inside the workspace.  `vec`: C's rows take 16-byte
 // stores.
 constexpr int kSumThreads = 256;
 __global__ void __launch_bounds__(kSumThreads)
@@ -2561,15 +2612,19 @@ hipError_t launch_dma(const GemmParams& p, bool ta, bool tb, int nbatch, hipStre
     return hipGetLastError();
 }
 
+// A slice's partial product: M rows of N floats, rounded up to 16 bytes.
+inline int slice_ld(int N) { return (N + 3) / 4 * 4; }
+inline int64_t slice_matrix(int M, int N) { return (int64_t)M * slice_ld(N); }
+
 // C = epi(op(A) op(B)) as `slices` products over kslice steps of K each, every
-// one to its own tile-padded matrix in `ws`, and a second launch that adds
-// them in slice order.  For outputs whose tiles leave most CUs idle.
+// one to its own matrix in `ws` (slice_matrix floats), and a second launch that
+// adds them in slice order.  For outputs whose tiles leave most CUs idle.
 template <class Cfg>
 hipError_t launch_sliced(const GemmParams& p, bool ta, bool tb, int slices, int kslice, float* ws,
                          hipStream_t stream) {
     static_assert(Cfg::SLICED != 0, "a K-slice configuration");
-    const int ldp = (p.N + Cfg::BN - 1) / Cfg::BN * Cfg::BN;
-    const int64_t slice = (int64_t)((p.M + Cfg::BM - 1) / Cfg::BM * Cfg::BM) * ldp;
+    const int ldp = slice_ld(p.N);
+    const int64_t slice = slice_matrix(p.M, p.N);
     GemmParams q = p;
     q.strideA = ta ? kslice * p.lda : kslice;
     q.strideB = tb ? kslice : kslice * p.ldb;
@@ -3311,7 +3366,7 @@ SlicePlan slice_plan(const GemmParams& p, bool transA, bool transB, int64_t batc
     const int bm = p.M <= 32 ? 32 : 64, bn = 64;
     const int64_t tiles_m = (p.M + bm - 1) / bm, tiles_n = (p.N + bn - 1) / bn;
     const int64_t tiles = tiles_m * tiles_n;
-    const double matrix = (double)tiles * bm * bn * sizeof(float);
+    const double matrix = (double)slice_matrix(p.M, p.N) * sizeof(float);
     const double per_step = bm == 32 ? 0.0082 : 0.0150;
     constexpr int64_t kCUs = 256;
     constexpr int kStep = 64;  // slices are whole K-tiles
@@ -3333,7 +3388,7 @@ SlicePlan slice_plan(const GemmParams& p, bool transA, bool transB, int64_t batc
             best_us = us;
             s.slices = (int)slices;
             s.kslice = (int)steps;
-            s.bytes = (size_t)slices * tiles * bm * bn * sizeof(float);
+            s.bytes = (size_t)slices * slice_matrix(p.M, p.N) * sizeof(float);
         }
     }
     return s;
@@ -3485,6 +3540,29 @@ hipError_t launch_group(const GroupJob* jobs, int n, hipStream_t stream) {
         }
     }
     return hipErrorInvalidValue;
+}
+
+hipError_t launch_weight_grad(const GemmParams& p, bool transA, bool transB, float* scratch,
+                              size_t scratch_bytes, hipStream_t stream) {
+    constexpr int64_t kBlocks = 512;  // two per CU
+    constexpr int kStep = 64;
+    const int bm = p.M <= 32 ? 32 : 64, bn = 64;
+    const int64_t tiles = (int64_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
+    const size_t matrix = (size_t)slice_matrix(p.M, p.N) * sizeof(float);
+    int64_t slices = std::max<int64_t>(1, kBlocks / tiles);
+    slices = std::min<int64_t>(slices, (int64_t)(scratch_bytes / matrix));
+    constexpr size_t kMaxMatrix = size_t(1) << 30;  // (the sum counts elements in 32 bits)
+    if (scratch != nullptr && slices >= 2 && matrix <= kMaxMatrix) {
+        SlicePlan s;
+        const int64_t steps = ((p.K + slices - 1) / slices + kStep - 1) / kStep * kStep;
+        s.kslice = (int)std::max<int64_t>(2 * kStep, steps);
+        s.slices = (p.K + s.kslice - 1) / s.kslice;
+        const hipError_t err = s.slices >= 2
+                                   ? launch_slice_plan(p, transA, transB, s, scratch, stream)
+                                   : hipErrorInvalidValue;
+        if (err != hipErrorInvalidValue) return err;
+    }
+    return launch_sgemm(p, transA, transB, 1, GemmKernel::Auto, stream);
 }
 
 hipError_t launch_sgemm(const GemmParams& p0, bool transA, bool transB,
