@@ -177,6 +177,85 @@ int device_scratch(float** out) {
     return FDL_SUCCESS;
 }
 
+// A training step after its forward product, for layers large enough that each
+// product is worth a launch of its own: one launch per product on the tiles that
+// suit it, the weight gradients over slices of the batch, and the parameter
+// updates last, in one launch, so that every product reads the old values.
+// Nothing is allocated: the loss's partial sums lie in dW1 and the slices'
+// partial products in dX, each before its own product writes it.
+int large_step_backward(const float* X, const int64_t* labels, int64_t B, int64_t I, int64_t Hd,
+                        int64_t Cc, float* W1, float* b1, float* W2, float* b2, float lr,
+                        float* H, float* logits, float* G2, float* G1, float* dW1, float* db1,
+                        float* dW2, float* db2, float* dX, float* loss, hipStream_t hs) {
+    auto product = [](int64_t M, int64_t N, int64_t K, const float* A, int64_t lda,
+                      const float* Bm, int64_t ldb, float* C, int epi) {
+        fdl::GemmParams p = shape_params(M, N, K);
+        p.A = A;
+        p.B = Bm;
+        p.C = C;
+        p.lda = lda;
+        p.ldb = ldb;
+        p.ldc = N;
+        p.epilogue = epi;
+        return p;
+    };
+    const bool aligned = (reinterpret_cast<uintptr_t>(dX) & 15u) == 0;
+    float* scratch = aligned ? dX : nullptr;
+    const size_t scratch_bytes = scratch ? (size_t)(B * I) * sizeof(float) : 0;
+    int st;
+    // logits, G2 = dL/dlogits, G1 = (G2 W2^T) * [H > 0] and the loss's partial sums
+    int64_t nparts = fdl::head_blocks(B);
+    int stride = (int)Cc + 1;
+    const float* part = dW1 + Cc;  // (the head's record: column sums of G2, then its loss)
+    if (fdl::head_supported(Hd, Cc) && nparts * stride <= I * Hd) {
+        st = check_hip(fdl::launch_mlp_head(H, W2, b2, labels, logits, G2, G1, dW1, B, Hd, Cc, hs),
+                       "mlp2_train_step head failed");
+        if (st) return st;
+    } else {
+        fdl::GemmParams z = product(B, Cc, Hd, H, Hd, W2, Cc, logits, fdl::EPI_BIAS);
+        z.bias = b2;
+        st = check_hip(fdl::launch_sgemm(z, false, false, 1, fdl::GemmKernel::Auto, hs, scratch,
+                                         scratch_bytes),
+                       "mlp2_train_step logits failed");
+        if (st) return st;
+        nparts = fdl::xent_parts(B, Cc);
+        stride = 1;
+        part = dW1;
+        st = check_hip(fdl::launch_xent_parts(logits, labels, dW1, G2, B, Cc, hs),
+                       "mlp2_train_step loss failed");
+        if (st) return st;
+        fdl::GemmParams g = product(B, Hd, Cc, G2, Cc, W2, Cc, G1, fdl::EPI_RELU_GRAD);
+        g.aux = H;
+        st = check_hip(fdl::launch_sgemm(g, false, true, 1, fdl::GemmKernel::Auto, hs),
+                       "mlp2_train_step G1 failed");
+        if (st) return st;
+    }
+    st = check_hip(fdl::launch_step_reduce(G1, db1, Hd, G2, db2, Cc, B, part, nparts, stride, loss,
+                                           hs),
+                   "mlp2_train_step reductions failed");
+    if (st) return st;
+    // dW2 = H^T G2, dW1 = X^T G1 (TN)
+    st = check_hip(fdl::launch_weight_grad(product(Hd, Cc, B, H, Hd, G2, Cc, dW2, fdl::EPI_NONE),
+                                           true, false, scratch, scratch_bytes, hs),
+                   "mlp2_train_step dW2 failed");
+    if (st) return st;
+    st = check_hip(fdl::launch_weight_grad(product(I, Hd, B, X, I, G1, Hd, dW1, fdl::EPI_NONE),
+                                           true, false, scratch, scratch_bytes, hs),
+                   "mlp2_train_step dW1 failed");
+    if (st) return st;
+    if (dX) {  // dX = G1 W1^T (NT)
+        st = check_hip(fdl::launch_sgemm(product(B, I, Hd, G1, Hd, W1, Hd, dX, fdl::EPI_NONE),
+                                         false, true, 1, fdl::GemmKernel::Auto, hs),
+                       "mlp2_train_step dX failed");
+        if (st) return st;
+    }
+    float* params[4] = {W1, b1, W2, b2};
+    const float* grads[4] = {dW1, db1, dW2, db2};
+    const int64_t sizes[4] = {I * Hd, Hd, Hd * Cc, Cc};
+    return check_hip(fdl::launch_sgd_multi(4, params, grads, sizes, lr, hs),
+                     "mlp2_train_step update failed");
+}
+
 }  // namespace
 
 extern "C" {
@@ -402,6 +481,22 @@ int fdl_mlp2_train_step(const float* X, const int64_t* labels, int64_t batch,
                        (dX ? fdl::head_dx_supported(B, I, Hd, Cc, H, W1)
                            : fdl::head_supported(Hd, Cc) &&
                                  fdl::head_blocks(B) * (Cc + 1) <= I * Hd);
+    const int64_t records = fdl::head_blocks(B);
+    const bool fused_head = fdl::head_supported(Hd, Cc) && records * (Cc + 1) <= I * Hd;
+    // Large layers take one launch per product instead of the grouped ones
+    // below, whose 32x32 tiles are for products too small for the GPU.  From
+    // how many multiply-adds in the first layer, by what the grouped form's
+    // head costs; measured (us, grouped / one launch per product): three
+    // launches 2048x784x256x10 61 / 72, 3000x1000x256x10 104 / 84,
+    // 4096x1024x256x32 158 / 97; four 600x784x700x10 66 / 81,
+    // 4096x400x300x12 130 / 97; six 512x784x512x100 57 / 61, 1024x200x700x20
+    // 81 / 59, 2048x784x1024x100 243 / 159, 3520x364x912x18 312 / 162.
+    // (dW1 has to hold the loss's partial sums.)
+    const double size = (double)B * (double)I * (double)Hd;
+    if (size >= (three ? 6.0e8 : fused_head ? 4.0e8 : 1.2e8) && I * Hd >= fdl::xent_parts(B, Cc)) {
+        return large_step_backward(X, labels, B, I, Hd, Cc, W1, b1, W2, b2, lr, H, logits, G2, G1,
+                                   dW1, db1, dW2, db2, dX, loss, hs);
+    }
     if (three) {
         if (dX) {
             st = check_hip(fdl::launch_mlp_head_dx(H, W2, b2, labels, W1, logits, G2, G1, dX, B,
@@ -440,8 +535,6 @@ int fdl_mlp2_train_step(const float* X, const int64_t* labels, int64_t batch,
     // head (launch 2), b2 is updated in launch 3 and W2 in launch 4; b1 is
     // read by launch 1 and updated in launch 3; W1 is read by launch 1 and by
     // the dX product (launch 3) and updated in launch 4.
-    const int64_t records = fdl::head_blocks(B);
-    const bool fused_head = fdl::head_supported(Hd, Cc) && records * (Cc + 1) <= I * Hd;
     if (fused_head) {
         // Launch 2: logits, loss shares, G2 and G1 = (G2 W2^T) * [H > 0].
         st = check_hip(fdl::launch_mlp_head(H, W2, b2, labels, logits, G2, G1, dW1, B, Hd, Cc,

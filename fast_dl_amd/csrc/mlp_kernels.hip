@@ -64,17 +64,19 @@ constexpr int kTallCols = 4;
 constexpr int64_t kColsumShort = 2048;
 
 template <bool VEC>
-__global__ void __launch_bounds__(kTallThreads)
-colsum_tall_kernel(const float* __restrict__ x, float* __restrict__ out,
-                   float* __restrict__ param, float lr, int64_t rows, int64_t cols) {
+__device__ __forceinline__ void colsum_tall_body(const float* __restrict__ x,
+                                                 float* __restrict__ out,
+                                                 float* __restrict__ param, float lr,
+                                                 int64_t rows, int64_t cols, int block,
+                                                 int nblocks) {
 #pragma clang fp contract(off)
     constexpr int V = kTallCols, kUnroll = 4;
     constexpr int kWaves = kTallThreads / 64;
     __shared__ float red[kWaves][V];
     // strips in order over XCDs (block b runs on XCD b % 8), each a contiguous range
-    const int64_t per = gridDim.x / 8, extra = gridDim.x % 8;
-    const int64_t xcd = blockIdx.x % 8;
-    const int64_t c0 = (xcd * per + min(xcd, extra) + blockIdx.x / 8) * V;
+    const int64_t per = nblocks / 8, extra = nblocks % 8;
+    const int64_t xcd = block % 8;
+    const int64_t c0 = (xcd * per + min(xcd, extra) + block / 8) * V;
     const float* col = x + c0;
     float s[V] = {};
     for (int64_t r0 = threadIdx.x; r0 < rows; r0 += (int64_t)kUnroll * kTallThreads) {
@@ -113,6 +115,44 @@ colsum_tall_kernel(const float* __restrict__ x, float* __restrict__ out,
         if (param) {
             const float step = lr * t;
             param[c] -= step;
+        }
+    }
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(kTallThreads)
+colsum_tall_kernel(const float* __restrict__ x, float* __restrict__ out,
+                   float* __restrict__ param, float lr, int64_t rows, int64_t cols) {
+    colsum_tall_body<VEC>(x, out, param, lr, rows, cols, blockIdx.x, gridDim.x);
+}
+
+// The reductions of a large training step in one launch: db1 and db2, the
+// column sums of G1 (blocks 0 .. n1 - 1) and of G2 (the next n2), and the loss, the sum of
+// nparts partial sums `stride` floats apart (the last block).
+template <bool VEC1, bool VEC2>
+__global__ void __launch_bounds__(kTallThreads)
+step_reduce_kernel(const float* __restrict__ G1, float* __restrict__ db1, int hidden, int n1,
+                   const float* __restrict__ G2, float* __restrict__ db2, int classes, int n2,
+                   int64_t rows, const float* __restrict__ part, int nparts, int stride,
+                   float* __restrict__ loss) {
+    const int block = blockIdx.x;
+    if (block < n1) {
+        colsum_tall_body<VEC1>(G1, db1, nullptr, 0.0f, rows, hidden, block, n1);
+    } else if (block < n1 + n2) {
+        colsum_tall_body<VEC2>(G2, db2, nullptr, 0.0f, rows, classes, block - n1, n2);
+    } else {
+        constexpr int kWaves = kTallThreads / 64;
+        __shared__ float red[kWaves];
+        float s = 0.0f;
+        for (int b = threadIdx.x; b < nparts; b += kTallThreads) s += part[(int64_t)b * stride];
+        s = wave_sum(s);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x / 64] = s;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            float t = red[0];
+#pragma unroll
+            for (int w = 1; w < kWaves; ++w) t += red[w];
+            loss[0] = t;
         }
     }
 }
@@ -813,17 +853,25 @@ struct SgdMulti {
     int64_t n[4];
 };
 
-// blockIdx.y selects the tensor; the x grid strides over the largest one.
-__global__ void sgd_multi_kernel(SgdMulti args, float lr) {
-#pragma clang fp contract(off)
+// blockIdx.y selects the tensor; the x grid strides over the largest one, 16
+// bytes per lane over each tensor's aligned body.
+__global__ void __launch_bounds__(kBlock) sgd_multi_kernel(SgdMulti args, OpSgd op) {
     const int t = blockIdx.y;
-    float* __restrict__ p = args.p[t];
-    const float* __restrict__ g = args.g[t];
-    const int64_t n = args.n[t];
-    for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < n;
-         idx += (int64_t)gridDim.x * blockDim.x) {
-        p[idx] -= lr * g[idx];
+    float* p = args.p[t];
+    const float* g = args.g[t];
+    const bool vec = ((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(g)) & 15u) == 0;
+    const int64_t n4 = vec ? args.n[t] / 4 : 0;
+    const int64_t first = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+    const int64_t step = (int64_t)gridDim.x * kBlock;
+    for (int64_t i = first; i < n4; i += step) {
+        const floatx4 vp = reinterpret_cast<const floatx4*>(p)[i];
+        const floatx4 vg = reinterpret_cast<const floatx4*>(g)[i];
+        floatx4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = op(vp[e], vg[e]);
+        reinterpret_cast<floatx4*>(p)[i] = r;
     }
+    for (int64_t i = 4 * n4 + first; i < args.n[t]; i += step) p[i] = op(p[i], g[i]);
 }
 
 // data[0 .. bytes) = 0: 16-byte stores over the aligned body, byte stores at
@@ -1024,7 +1072,31 @@ hipError_t launch_sgd_multi(int count, float* const* params,
     }
     if (nmax == 0) return hipSuccess;
     hipLaunchKernelGGL(sgd_multi_kernel, dim3(grid_for(nmax, 4), count),
-                       dim3(kBlock), 0, stream, args, lr);
+                       dim3(kBlock), 0, stream, args, OpSgd{lr});
+    return hipGetLastError();
+}
+
+hipError_t launch_step_reduce(const float* G1, float* db1, int64_t hidden, const float* G2,
+                              float* db2, int64_t classes, int64_t rows, const float* part,
+                              int64_t nparts, int stride, float* loss, hipStream_t stream) {
+    auto vec = [](const float* x, int64_t cols) {
+        return cols % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+    };
+    const int n1 = (int)((hidden + kTallCols - 1) / kTallCols);
+    const int n2 = (int)((classes + kTallCols - 1) / kTallCols);
+    const dim3 grid(n1 + n2 + 1);
+#define FDL_STEP_REDUCE(V1, V2)                                                                  \
+    hipLaunchKernelGGL((step_reduce_kernel<V1, V2>), grid, dim3(kTallThreads), 0, stream, G1,   \
+                       db1, (int)hidden, n1, G2, db2, (int)classes, n2, rows, part, (int)nparts, \
+                       stride, loss)
+    if (vec(G1, hidden)) {
+        if (vec(G2, classes)) FDL_STEP_REDUCE(true, true);
+        else FDL_STEP_REDUCE(true, false);
+    } else {
+        if (vec(G2, classes)) FDL_STEP_REDUCE(false, true);
+        else FDL_STEP_REDUCE(false, false);
+    }
+#undef FDL_STEP_REDUCE
     return hipGetLastError();
 }
 

@@ -371,6 +371,33 @@ hipError_t launch_softmax(const float* in, float* out, int64_t rows, int64_t col
     });
 }
 
+int64_t xent_parts(int64_t batch, int64_t classes) {
+    if (classes > kMaxRegCols) return std::min<int64_t>(batch, kMaxRowBlocks);
+    int64_t blocks = 0;
+    (void)with_row_regs(classes, false, [&](auto row) {
+        constexpr int kPerBlock = kRowThreads / decltype(row)::G;
+        blocks = std::min<int64_t>((batch + kPerBlock - 1) / kPerBlock, kMaxRowBlocks);
+        return hipSuccess;
+    });
+    return blocks;
+}
+
+hipError_t launch_xent_parts(const float* logits, const int64_t* labels, float* part, float* grad,
+                             int64_t batch, int64_t classes, hipStream_t stream) {
+    const dim3 grid((unsigned)xent_parts(batch, classes));
+    if (classes > kMaxRegCols) {
+        hipLaunchKernelGGL(xent_wide_kernel, grid, dim3(kOneBlockThreads), 0, stream, logits,
+                           labels, part, grad, batch, classes, (int64_t)0);
+        return hipGetLastError();
+    }
+    return with_row_regs(classes, rows_vec4(logits, grad, classes), [&](auto row) {
+        using Row = decltype(row);
+        hipLaunchKernelGGL((xent_kernel<Row>), grid, dim3(kRowThreads), 0, stream, logits, labels,
+                           part, grad, batch, (int)classes, (int64_t)0);
+        return hipGetLastError();
+    });
+}
+
 // Many blocks and a second launch that adds their loss sums, unless one block
 // takes the batch in few rounds of its 1024 threads: three of up to 4 columns
 // per thread (about 1 us each: 513 x 10 in three rounds 4.5 us against 4.8 us

@@ -284,7 +284,9 @@ int fdl_sgd_update(float* param, const float* grad, float lr, int64_t n,
  * classes <= 32 and hidden <= 512, and ceil(batch / 8) * (classes + 1) <=
  * in_features * hidden: then dW1 holds per-block partial sums of the loss
  * and db2 until the last launch writes the weight gradient into it.
- * Otherwise it is 6 launches.
+ * Otherwise it is 6 launches.  Large layers take one launch per product, and
+ * one for all updates; dX then holds partial sums of the weight gradients
+ * until its own product writes it.
  */
 int fdl_mlp2_train_step(const float* X, const int64_t* labels,
                         int64_t batch, int64_t in_features,
