@@ -6,6 +6,7 @@ Compiles, in-tree, with hipcc for gfx950 only:
   ``include/fastdl_gemm.h`` and ``include/fastdl_data.h``;
 * ``fast_dl_amd/libfastdl.so`` -- the C++ ``dl::`` tensor/ops/nn API
   (``include/dl``) hosted on the HIP runtime, linked against the former;
+* ``fast_dl_amd/_fastcall.so`` -- the CPython side of ``fast_dl_amd.capi``'s calls;
 * the C++ API test programs under ``tests/cpp`` (``tests/cpp/bin``).
 
 Every call rebuilds everything (the driver uses this as the "does it build"
@@ -19,6 +20,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -112,6 +114,16 @@ def build_dl_library() -> str | None:
     return out
 
 
+def build_python_module() -> str:
+    src = os.path.join(CSRC, "python", "fastcall.cpp")
+    out = os.path.join(PKG, "_fastcall.so")
+    tmp = out + ".tmp"
+    _run([HOST_CXX, "-O2", "-fPIC", "-std=c++17", "-Wall", "-shared", "-I", INCLUDE,
+          "-I", sysconfig.get_paths()["include"], src, "-o", tmp])
+    os.replace(tmp, out)
+    return out
+
+
 def build_cpp_tests() -> list[str]:
     test_dir = os.path.join(ROOT, "tests", "cpp")
     srcs = sorted(glob.glob(os.path.join(test_dir, "*.cpp")))
@@ -140,6 +152,9 @@ def build_all(verbose: bool = True) -> None:
     lib = build_gemm_library()
     if verbose:
         print(f"built {lib}")
+    module = build_python_module()
+    if verbose:
+        print(f"built {module}")
     dl = build_dl_library()
     if dl and verbose:
         print(f"built {dl}")

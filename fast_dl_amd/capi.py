@@ -1,6 +1,8 @@
-"""ctypes binding of ``include/fastdl_gemm.h``.
+"""Binding of ``include/fastdl_gemm.h`` and ``include/fastdl_data.h``.
 
-Every function takes raw device addresses (ints, e.g. ``tensor.data_ptr()``)
+ctypes loads the library and declares every entry point; the calls a program
+repeats go through ``_fastcall``, the same calls without ctypes' conversions,
+where that module is built.  Every function takes raw device addresses (ints, e.g. ``tensor.data_ptr()``)
 and a raw ``hipStream_t`` (int, e.g. ``torch.cuda.current_stream().cuda_stream``,
 0 for the null stream).  Non-zero statuses raise :class:`FdlError` carrying
 the library's own message.
@@ -9,6 +11,11 @@ from __future__ import annotations
 
 import ctypes
 import os
+
+try:
+    from fast_dl_amd import _fastcall
+except ImportError:  # the library alone was built: the ctypes calls serve
+    _fastcall = None
 
 OP_N, OP_T = 0, 1
 EPILOGUE_NONE, EPILOGUE_BIAS, EPILOGUE_BIAS_RELU, EPILOGUE_RELU, EPILOGUE_RELU_GRAD = range(5)
@@ -98,8 +105,14 @@ def load_library() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+        if _fastcall is not None:
+            _fastcall.set_address(name, ctypes.cast(fn, _vp).value)
     _LIB = lib
     return lib
+
+
+def _fail(name: str, status: int):
+    raise FdlError(name, status, load_library().fdl_last_error().decode())
 
 
 def _checked(name: str):
@@ -107,10 +120,11 @@ def _checked(name: str):
         lib = load_library()
         status = getattr(lib, name)(*args)
         if status != 0:
-            raise FdlError(name, status, lib.fdl_last_error().decode())
+            _fail(name, status)
         return status
     call.__name__ = name
-    return call
+    fast = _fastcall.bind(name, call, _fail) if _fastcall is not None else None
+    return call if fast is None else fast
 
 
 sgemm_ex = _checked("fdl_sgemm_ex")
