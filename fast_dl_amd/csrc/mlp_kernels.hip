@@ -569,7 +569,7 @@ __device__ __forceinline__ float row16_sum(float x) {
 //     LDS and wave 0 adds them in wave order, adds b2 after the sum (as
 //     linear_cpu, tests/tensor/linear_tensor_test.cpp:17-25), and takes the
 //     softmax of each row over the 16 lanes of a DPP row: G2 as
-//     softmax_xent_kernel (legacy SoftmaxCrossEntropyLoss,
+//     xent_kernel (row_kernels.hip; legacy SoftmaxCrossEntropyLoss,
 //     legacy/src/ops/SoftmaxCrossEntropyLoss.cpp:39-51).  The loss is left to
 //     head_finalize_body, which reads the stored logits.
 //   G1 = (G2 W2^T) * [H > 0] (legacy/src/ops/Layers.cpp:36 through the ReLU
