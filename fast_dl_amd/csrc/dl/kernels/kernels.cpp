@@ -18,19 +18,35 @@
 
 namespace dl::detail {
 
+namespace {
+
+// Whether work on `stream` is being recorded into a graph (or the runtime cannot say).
+bool recording(void* stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    const hipError_t before = hipPeekAtLastError();
+    const hipError_t err = hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status);
+    if (err != hipSuccess && before == hipSuccess) (void)hipGetLastError();
+    return err != hipSuccess || status != hipStreamCaptureStatusNone;
+}
+
+}  // namespace
+
 int sgemm_auto(int transA, int transB, int64_t M, int64_t N, int64_t K, const float* A,
                int64_t lda, int64_t strideA, const float* B, int64_t ldb, int64_t strideB,
                float* C, int64_t ldc, int64_t strideC, int64_t batch, const float* bias,
                const float* aux, int epilogue, void* stream) {
     const size_t bytes = fdl_sgemm_workspace_size(transA, transB, M, N, K, batch);
-    if (bytes == 0) {
+    int device = 0;
+    BlockCache& cache = device_block_cache();
+    void* ws = nullptr;
+    if (bytes > 0 && !recording(stream)) {
+        hip::check(hipGetDevice(&device), "cudaGetDevice failed");
+        ws = cache.try_acquire(device, bytes, stream);
+    }
+    if (!ws) {
         return fdl_sgemm_ex(transA, transB, M, N, K, A, lda, strideA, B, ldb, strideB, C, ldc,
                             strideC, batch, bias, aux, epilogue, stream);
     }
-    int device = 0;
-    hip::check(hipGetDevice(&device), "cudaGetDevice failed");
-    BlockCache& cache = device_block_cache();
-    void* ws = cache.acquire(device, bytes, stream);
     const int status = fdl_sgemm_ex_ws(transA, transB, M, N, K, A, lda, strideA, B, ldb,
                                        strideB, C, ldc, strideC, batch, bias, aux, epilogue, ws,
                                        bytes, stream);

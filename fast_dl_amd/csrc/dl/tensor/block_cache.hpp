@@ -71,6 +71,12 @@ public:
     // std::runtime_error("cudaMalloc failed: ...") when the device has no
     // memory left even after every cached block was returned to it.
     void* acquire(int device, std::size_t bytes, void* stream) {
+        if (void* p = try_acquire(device, bytes, stream)) return p;
+        throw std::runtime_error("cudaMalloc failed: " + be_.last_error());
+    }
+
+    // As acquire, for a block its caller can do without: null instead of throwing.
+    void* try_acquire(int device, std::size_t bytes, void* stream) {
         const std::size_t sz = round(bytes);
         {
             std::lock_guard<std::mutex> lock(mu_);
@@ -82,8 +88,7 @@ public:
         if (be_.alloc(device, sz, &p)) return p;
         // Return every cached block of this device to the runtime and retry once.
         release_all(device);
-        if (be_.alloc(device, sz, &p)) return p;
-        throw std::runtime_error("cudaMalloc failed: " + be_.last_error());
+        return be_.alloc(device, sz, &p) ? p : nullptr;
     }
 
     // Gives back a block allocated on `home`.  `uses` are the other streams

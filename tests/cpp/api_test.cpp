@@ -5,6 +5,8 @@
 #include <dl/dl.hpp>
 #include <dl/kernels/kernels.hpp>
 
+#include <fastdl_gemm.h>
+
 #include <hip/hip_runtime_api.h>
 
 #include <cmath>
@@ -574,6 +576,84 @@ int main() {
         auto b = dl::Tensor::from_host<float>(hb, dl::Shape({k, n}), kDev);
         auto c = dl::ops::matmul(a, b);
         return close(c.to_host<float>(), host_gemm(ha, hb, m, n, k), 1e-4f);
+    });
+
+    // 33 x 200 x 4096 runs as slices of K when it gets a workspace; without memory for
+    // one it runs in a single pass, and the failed allocation surfaces nowhere.
+    run("matmul_without_memory_for_its_workspace", [] {
+        const int m = 33, n = 200, k = 4096;
+        const bool sliced = fdl_sgemm_workspace_size(FDL_OP_N, FDL_OP_N, m, n, k, 1) > 0;
+        const auto ha = randv(m * k, 61), hb = randv(k * n, 62);
+        const auto want = host_gemm(ha, hb, m, n, k);
+        dl::Stream s(kDev);  // a stream with no cached block
+        dl::StreamGuard guard(s);
+        auto a = dl::Tensor::from_host<float>(ha, dl::Shape({m, k}), kDev);
+        auto b = dl::Tensor::from_host<float>(hb, dl::Shape({k, n}), kDev);
+        dl::Tensor c(dl::Shape({m, n}), dl::DType::Float32, kDev);
+        dl::detail::inject_alloc_failures(2);  // the allocation and its retry
+        const std::string why = message_of([&] {
+            dl::kernels::gemm_ex(dl::kernels::Transpose::No, dl::kernels::Transpose::No, m, n, k,
+                                 static_cast<const float*>(a.data()), k, 0,
+                                 static_cast<const float*>(b.data()), n, 0,
+                                 static_cast<float*>(c.data()), n, 0, 1, nullptr, nullptr,
+                                 dl::kernels::Epilogue::None, dl::kernels::GemmAlgo::Auto,
+                                 s.handle());
+        });
+        dl::detail::inject_alloc_failures(0);
+        if (!why.empty()) std::cout << why << std::endl;
+        return sliced && why.empty() && close(c.to_host<float>(), want, 1e-4f);
+    });
+
+    // The same product captured into a graph: nothing is allocated during the capture
+    // and the graph holds no block of the cache, so replays stay right while the blocks
+    // that eager work left in the cache go to other tensors.
+    run("sliced_matmul_captured_in_a_graph_replays", [] {
+        const int m = 33, n = 200, k = 4096;
+        const auto ha = randv(m * k, 63), hb = randv(k * n, 64);
+        const auto want = host_gemm(ha, hb, m, n, k);
+        const std::size_t bytes = fdl_sgemm_workspace_size(FDL_OP_N, FDL_OP_N, m, n, k, 1);
+        bool ok = bytes > 0;
+        for (const bool warm : {false, true}) {
+            dl::Stream s(kDev);
+            dl::StreamGuard guard(s);
+            const hipStream_t hs = static_cast<hipStream_t>(s.handle());
+            auto a = dl::Tensor::from_host<float>(ha, dl::Shape({m, k}), kDev);
+            auto b = dl::Tensor::from_host<float>(hb, dl::Shape({k, n}), kDev);
+            dl::Tensor c(dl::Shape({m, n}), dl::DType::Float32, kDev);
+            const auto product = [&] {
+                dl::kernels::gemm_ex(dl::kernels::Transpose::No, dl::kernels::Transpose::No, m, n,
+                                     k, static_cast<const float*>(a.data()), k, 0,
+                                     static_cast<const float*>(b.data()), n, 0,
+                                     static_cast<float*>(c.data()), n, 0, 1, nullptr, nullptr,
+                                     dl::kernels::Epilogue::None, dl::kernels::GemmAlgo::Auto, hs);
+            };
+            if (warm) product();  // leaves a workspace in the cache
+            s.synchronize();
+            hipGraph_t graph = nullptr;
+            hipGraphExec_t exec = nullptr;
+            ok = hipStreamBeginCapture(hs, hipStreamCaptureModeThreadLocal) == hipSuccess && ok;
+            const std::string why = message_of(product);
+            ok = hipStreamEndCapture(hs, &graph) == hipSuccess && ok && why.empty();
+            if (!why.empty()) std::cout << why << std::endl;
+            ok = ok && hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess;
+            // a tensor of the workspace's size: the cached block, if there is one
+            dl::Tensor other(dl::Shape({static_cast<int64_t>(bytes / 4)}), dl::DType::Float32,
+                             kDev);
+            const std::vector<float> mark(bytes / 4, 7.0f);
+            const std::vector<float> nan_c(m * n, std::nanf(""));
+            for (int rep = 0; rep < 3 && ok; ++rep) {
+                other.copy_from_host(mark.data(), bytes);
+                c.copy_from_host(nan_c.data(), nan_c.size() * sizeof(float));
+                ok = hipGraphLaunch(exec, hs) == hipSuccess &&
+                     hipStreamSynchronize(hs) == hipSuccess;
+                ok = ok && close(c.to_host<float>(), want, 1e-4f) &&
+                     other.to_host<float>() == mark;
+            }
+            if (exec) ok = hipGraphExecDestroy(exec) == hipSuccess && ok;
+            if (graph) ok = hipGraphDestroy(graph) == hipSuccess && ok;
+            (void)hipGetLastError();
+        }
+        return ok;
     });
 
     std::cout << "api_test : " << (g_failures == 0 ? "passed" : "not passed") << std::endl;

@@ -207,6 +207,17 @@ int main() {
         return false;
     });
 
+    // A block its caller can do without: the same retry, then null.
+    check("try_acquire_after_failed_retry_is_null", [] {
+        FakeBackend be;
+        BlockCache c(be);
+        be.fail = 2;
+        if (c.try_acquire(0, 512, nullptr) != nullptr || be.allocs != 2) return false;
+        void* a = c.try_acquire(0, 512, nullptr);
+        c.release(0, 512, a, nullptr, {});
+        return a != nullptr && c.try_acquire(0, 512, nullptr) == a && be.allocs == 3;
+    });
+
     std::cout << (g_failures ? "block_cache_test : not passed" : "block_cache_test : passed")
               << std::endl;
     return g_failures;
