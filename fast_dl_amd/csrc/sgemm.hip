@@ -265,11 +265,17 @@ struct TileLoader {
 //
 // Stores go through a buffer descriptor based at the wave's corner, each lane's
 // column and half-row as a 32-bit offset and the row part wave-uniform (a
-// scalar offset), so a store costs no address arithmetic and no wait; blocks
-// on C's edge test each element's row and column.  `bias_pre`, when given,
-// holds this lane's bias value of each column block, fetched before the K
-// loop.  The per-element path below it serves the epilogue that updates a
-// parameter and rows too long for 32-bit offsets.
+// scalar offset), so a store costs no address arithmetic and no wait.  Blocks
+// on C's edge add the row part to the lane's offset, which the descriptor's
+// size is checked against, so stores past C's last row are dropped without a
+// branch; lanes past its last column skip a column block.  `bias_pre`, when
+// given, holds this lane's bias value of each column block, fetched before the
+// K loop.  The per-element path below it serves the epilogue that updates a
+// parameter, rows too long for 32-bit offsets, and the edge blocks of waves of
+// 16 or more 32x32 blocks (kWhole).  Their accumulators alone take 256 of a
+// lane's 512 registers, and a second form of the store code spilled 2 to 6
+// more around the K loop (4096^3 915-922 us; without spills 910, as before
+// edge blocks had a form of their own).
 constexpr int kBufferWord3Store = 0x00020000;  // raw-buffer descriptor word 3 (gfx9 family)
 
 // STREAM = 1: the fast path's stores are non-temporal (buffer store `nt`), for
@@ -279,74 +285,77 @@ template <int FM, int FN, int STREAM = 0>
 __device__ __forceinline__ void store_wave_tile(floatx16 (&acc)[FM][FN], const GemmParams& p,
                                                 int64_t bz, int mw, int nw, int half,
                                                 int l32, const float* bias_pre = nullptr) {
+    constexpr bool kWhole = FM * FN >= 16;
+    // mw and nw are wave-uniform by construction; saying so keeps the
+    // descriptors in scalar registers.
+    const int mwu = __builtin_amdgcn_readfirstlane(mw);
+    const int nwu = __builtin_amdgcn_readfirstlane(nw);
+    const int rows = p.M - mwu;  // (edge blocks: rows and columns inside C)
+    const int cols = p.N - nwu;
+    const bool inside = rows >= FM * 32 && cols >= FN * 32;
     // Byte offsets stay below 2^31: (FM * 32 rows) * ldc * 4 bytes.
-    if (p.epilogue != EPI_SGD && p.ldc < (int64_t(1) << 29) / (FM * 32)) {
+    // (Where the tests stand matters to the compiler's register allocation: with
+    // the scalar copies in this one CfgDma256W4 spills a register, and with the
+    // return below ahead of it CfgDma256 and CfgTiled256 spill 80 to 90.)
+    if (p.epilogue != EPI_SGD && (!kWhole || (mw + FM * 32 <= p.M && nw + FN * 32 <= p.N)) &&
+        p.ldc < (int64_t(1) << 29) / (FM * 32)) {
+        if (rows <= 0 || cols <= 0) return;
         const int epi = p.epilogue;
         const bool has_bias = epi == EPI_BIAS || epi == EPI_BIAS_RELU;
         const bool relu = epi == EPI_BIAS_RELU || epi == EPI_RELU;
-        // mw and nw are wave-uniform by construction; saying so keeps the
-        // descriptors in scalar registers.
-        const int mwu = __builtin_amdgcn_readfirstlane(mw);
-        const int nwu = __builtin_amdgcn_readfirstlane(nw);
-        const int rows = p.M - mwu;  // (edge blocks: rows and columns inside C)
-        const int cols = p.N - nwu;
-        if (rows <= 0 || cols <= 0) return;
-        const bool inside = rows >= FM * 32 && cols >= FN * 32;
         const int64_t corner = bz * p.strideC + (int64_t)mwu * p.ldc + nwu;
-        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-            p.C + corner, (short)0, -1, kBufferWord3Store);
         const int ldc = (int)p.ldc;
-        const uint32_t lane_off = (uint32_t)((4 * half) * ldc + l32) * 4u;
-        // Element r of block (mi, ni) is row mi * 32 + 8 (r / 4) + r % 4 + 4 half,
-        // column ni * 32 + l32 of the wave's tile.
-        auto put = [&](auto edge, int mi, int ni, int r, float v) __attribute__((always_inline)) {
-            const int row = mi * 32 + 8 * (r >> 2) + (r & 3);
-            if (!decltype(edge)::value || (row + 4 * half < rows && ni * 32 + l32 < cols)) {
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc,
-                                                      (int)lane_off, (row * ldc + ni * 32) * 4,
-                                                      STREAM ? 2 : 0);  // 2: nt
-            }
-        };
+        const int bytes = min(rows, FM * 32) * ldc * 4;
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            p.C + corner, (short)0, bytes, kBufferWord3Store);
+        const int lane_off = ((4 * half) * ldc + l32) * 4;
         using Edge = std::true_type;
         using Inside = std::false_type;
+        // Element r of block (mi, ni) is row mi * 32 + 8 (r / 4) + r % 4 + 4 half,
+        // column ni * 32 + l32 of the wave's tile.
+        auto row_off = [&](int mi, int r) __attribute__((always_inline)) {
+            return (mi * 32 + 8 * (r >> 2) + (r & 3)) * ldc * 4;
+        };
+        auto put = [&](auto edge, int mi, int ni, int r, float v) __attribute__((always_inline)) {
+            constexpr bool kEdge = decltype(edge)::value;
+            const int off = row_off(mi, r) + ni * 128;
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc,
+                                                  kEdge ? lane_off + off : lane_off,
+                                                  kEdge ? 0 : off, STREAM ? 2 : 0);  // 2: nt
+        };
         if (epi == EPI_RELU_GRAD) {
             // The ReLU-backward mask: each 32x32 block's 16 mask values loaded
-            // together ahead of its stores, two blocks at a time (one by one, each
-            // load waits out the stores before it).  2048x1024x100 14.2 -> 9.4 us,
-            // 4096x4096x256 200 -> 87 us.
+            // together ahead of its stores (one by one, each load waits out the
+            // stores before it).  2048x1024x100 11.4 -> 8.9 us, 4096x4096x256
+            // 155 -> 89 us.
             const __amdgpu_buffer_rsrc_t raux = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<float*>(p.aux) + corner, (short)0, -1, kBufferWord3Store);
-            constexpr int kBlocks = FM * FN;
-            constexpr int kPair = kBlocks > 1 ? 2 : 1;
+                const_cast<float*>(p.aux) + corner, (short)0, bytes, kBufferWord3Store);
             auto masked = [&](auto edge) __attribute__((always_inline)) {
+                constexpr bool kEdge = decltype(edge)::value;
 #pragma unroll
-                for (int b0 = 0; b0 < kBlocks; b0 += kPair) {
-                    float mask[kPair][16];
+                for (int ni = 0; ni < FN; ++ni) {
+                    if (kEdge && ni * 32 + l32 >= cols) continue;
 #pragma unroll
-                    for (int b = 0; b < kPair; ++b)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            const int mi = (b0 + b) % FM, ni = (b0 + b) / FM;
-                            const int row = mi * 32 + 8 * (r >> 2) + (r & 3);
-                            int off = (int)lane_off, base = (row * ldc + ni * 32) * 4;
-                            if constexpr (decltype(edge)::value) {  // clamped into C
-                                off = (min(row + 4 * half, rows - 1) * ldc +
-                                       min(ni * 32 + l32, cols - 1)) * 4;
-                                base = 0;
-                            }
-                            mask[b][r] = __builtin_bit_cast(
-                                float, __builtin_amdgcn_raw_buffer_load_b32(raux, off, base, 0));
-                        }
-#pragma unroll
-                    for (int b = 0; b < kPair; ++b)
+                    for (int mi = 0; mi < FM; ++mi) {
+                        float mask[16];
 #pragma unroll
                         for (int r = 0; r < 16; ++r) {
-                            const int mi = (b0 + b) % FM, ni = (b0 + b) / FM;
-                            put(edge, mi, ni, r, mask[b][r] > 0.0f ? acc[mi][ni][r] : 0.0f);
+                            const int off = row_off(mi, r) + ni * 128;
+                            mask[r] = __builtin_bit_cast(
+                                float, __builtin_amdgcn_raw_buffer_load_b32(
+                                           raux, kEdge ? lane_off + off : lane_off,
+                                           kEdge ? 0 : off, 0));
                         }
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            put(edge, mi, ni, r, mask[r] > 0.0f ? acc[mi][ni][r] : 0.0f);
+                        }
+                    }
                 }
             };
-            if (inside) {
+            if constexpr (kWhole) {
+                masked(Inside{});
+            } else if (inside) {
                 masked(Inside{});
             } else {
                 masked(Edge{});
@@ -363,19 +372,25 @@ __device__ __forceinline__ void store_wave_tile(floatx16 (&acc)[FM][FN], const G
         // One uniform branch on the epilogue, then straight-line stores.
         auto store_all = [&](auto edge, auto op) __attribute__((always_inline)) {
 #pragma unroll
-            for (int ni = 0; ni < FN; ++ni)
+            for (int ni = 0; ni < FN; ++ni) {
+                if (decltype(edge)::value && ni * 32 + l32 >= cols) continue;
 #pragma unroll
                 for (int mi = 0; mi < FM; ++mi)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) put(edge, mi, ni, r, op(acc[mi][ni][r], bj[ni]));
+            }
         };
-        if (!inside) {
-            // (one copy of the code: the epilogue by selects)
-            store_all(Edge{}, [&](float v, float b) {
-                v = has_bias ? v + b : v;
-                return relu ? fmaxf(0.0f, v) : v;
-            });
-        } else if (has_bias && relu) {
+        if constexpr (!kWhole) {
+            if (!inside) {
+                // (one copy of the code: the epilogue by selects)
+                store_all(Edge{}, [&](float v, float b) {
+                    v = has_bias ? v + b : v;
+                    return relu ? fmaxf(0.0f, v) : v;
+                });
+                return;
+            }
+        }
+        if (has_bias && relu) {
             store_all(Inside{}, [](float v, float b) { return fmaxf(0.0f, v + b); });
         } else if (has_bias) {
             store_all(Inside{}, [](float v, float b) { return v + b; });
