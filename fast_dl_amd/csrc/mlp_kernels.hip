@@ -128,7 +128,8 @@ colsum_tall_kernel(const float* __restrict__ x, float* __restrict__ out,
 
 // The reductions of a large training step in one launch: db1 and db2, the
 // column sums of G1 (blocks 0 .. n1 - 1) and of G2 (the next n2), and the loss, the sum of
-// nparts partial sums `stride` floats apart (the last block).
+// nparts partial sums `stride` floats apart (the last block).  n1 or n2 may be
+// 0: that sum has a launch of its own.
 template <bool VEC1, bool VEC2>
 __global__ void __launch_bounds__(kTallThreads)
 step_reduce_kernel(const float* __restrict__ G1, float* __restrict__ db1, int hidden, int n1,
@@ -1082,8 +1083,19 @@ hipError_t launch_step_reduce(const float* G1, float* db1, int64_t hidden, const
     auto vec = [](const float* x, int64_t cols) {
         return cols % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
     };
-    const int n1 = (int)((hidden + kTallCols - 1) / kTallCols);
-    const int n2 = (int)((classes + kTallCols - 1) / kTallCols);
+    // Sums wider than the strips are good for go to launch_colsum (a launch also
+    // holds at most 2^32 threads, 2^24 columns in strips).
+    constexpr int64_t kMaxCols = 2048;
+    const int n1 = hidden <= kMaxCols ? (int)((hidden + kTallCols - 1) / kTallCols) : 0;
+    const int n2 = classes <= kMaxCols ? (int)((classes + kTallCols - 1) / kTallCols) : 0;
+    if (n1 == 0) {
+        const hipError_t err = launch_colsum(G1, db1, rows, hidden, stream);
+        if (err != hipSuccess) return err;
+    }
+    if (n2 == 0) {
+        const hipError_t err = launch_colsum(G2, db2, rows, classes, stream);
+        if (err != hipSuccess) return err;
+    }
     const dim3 grid(n1 + n2 + 1);
 #define FDL_STEP_REDUCE(V1, V2)                                                                  \
     hipLaunchKernelGGL((step_reduce_kernel<V1, V2>), grid, dim3(kTallThreads), 0, stream, G1,   \

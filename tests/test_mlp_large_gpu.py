@@ -82,3 +82,46 @@ def test_large_step_repeats_bit_for_bit(device):
     say("large step twice")
     a, b = (_step(X, labels, params, 0) for _ in range(2))
     assert all(np.array_equal(a[k], b[k]) for k in a)
+
+
+@pytest.mark.parametrize("B,I,Hd,C", [(2, 4, (1 << 24) + 8, 3), (130, 260, 4100, 40),
+                                      (64, 800, 2500, 2052)])
+def test_large_step_wide_layers(device, B, I, Hd, C):
+    """Bias gradients wider than the strips of the reduction launch take their own."""
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(B + Hd)
+
+    def rand(*shape, scale=1.0):
+        return torch.randn(*shape, generator=g, device="cuda") * scale
+
+    X, labels = rand(B, I), torch.arange(B, device="cuda") % C
+    W1, b1, W2, b2 = rand(I, Hd, scale=I ** -0.5), rand(Hd), rand(Hd, C, scale=Hd ** -0.5), rand(C)
+    new = {"W1": W1.clone(), "b1": b1.clone(), "W2": W2.clone(), "b2": b2.clone()}
+    out = {n: torch.full(s, float("nan"), device="cuda")
+           for n, s in dict(H=(B, Hd), logits=(B, C), G2=(B, C), G1=(B, Hd), dW1=(I, Hd),
+                            db1=(Hd,), dW2=(Hd, C), db2=(C,), dX=(B, I), loss=(1,)).items()}
+    say(f"large step, wide layers B={B} I={I} H={Hd} C={C}")
+    capi.mlp2_train_step(X.data_ptr(), labels.data_ptr(), B, I, Hd, C,
+                         *(t.data_ptr() for t in new.values()), LR,
+                         *(t.data_ptr() for t in out.values()), stream())
+    # fp64, from the step's own H and G1 masks on
+    H = out["H"].double()
+    assert torch.allclose(H, (X.double() @ W1.double() + b1).clamp_min(0), rtol=1e-5, atol=1e-5)
+    logits = H @ W2.double() + b2
+    p = torch.softmax(logits, 1)
+    p[torch.arange(B), labels] -= 1.0
+    G2 = p / B
+    G1 = (G2 @ W2.double().t().contiguous()) * (H > 0)
+    want = {"G2": G2, "G1": G1, "db2": G2.sum(0), "db1": G1.sum(0),
+            "dW2": H.t().contiguous() @ G2, "dW1": X.double().t().contiguous() @ G1,
+            "dX": G1 @ W1.double().t().contiguous()}
+    # rounding errors of a sum of n terms add like a random walk's steps, eps * sqrt(n) / 3
+    # of its norm at most; the gradients of logits pass theirs on
+    tol = 5e-6 + 4e-8 * np.sqrt(max(B, I, Hd, C))
+    for name, w in want.items():
+        err = (out[name].double() - w).norm() / w.norm()
+        assert err <= tol, f"{name}: {err:.2e}"
+    for name, w, dw in (("W1", W1, "dW1"), ("b1", b1, "db1"), ("W2", W2, "dW2"), ("b2", b2, "db2")):
+        step = LR * out[dw]
+        assert torch.equal(new[name], w - step)
