@@ -55,13 +55,43 @@ __device__ __forceinline__ float wave_sum(float v) {
 // one per nanosecond whatever the width of the strip, so narrow strips on many
 // CUs win; the blocks whose strips share a 128-byte line are numbered onto one
 // XCD, whose L2 then fetches the line once (without that 60000 x 256 took 122
-// us, as eight fetches of everything).  60000 x 256: 154 -> 53 us, 60000 x 1024:
-// 242 -> 103 us, 4096 x 1024: 12.4 -> 8.0 us; wider strips (8, 16 and 32
-// columns) 99, 107 and 112 us at 60000 x 256.  Up to kColsumShort rows
-// colsum_kernel's one round trip is faster (1024 x 256: 2.9 against 3.1 us).
+// us, as eight fetches of everything).  60000 x 256: 148 -> 55 us, 60000 x 1024:
+// 151 -> 98 us, 4096 x 512: 8.0 -> 6.3 us; wider strips (8, 16 and 32
+// columns) 99, 107 and 112 us at 60000 x 256.
 constexpr int kTallThreads = 1024;
 constexpr int kTallCols = 4;
-constexpr int64_t kColsumShort = 2048;
+
+// Whether rows of `cols` floats from x take 16-byte loads.
+inline bool vec_rows(const float* x, int64_t cols) {
+    return cols % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+}
+
+// Whether the strips beat colsum_kernel's 32-column blocks, which read whole
+// lines but leave CUs idle below 8192 columns.  Measured (us, blocks / strips):
+// * Up to 2048 rows the blocks' one round trip wins (1024 x 256 2.9 / 3.1).
+// * Up to 1024 columns every strip has a CU of its own: 4096 x 1000 13.3 / 7.9,
+//   30000 x 512 76 / 41; only wide matrices of few rows lose (2049 x 1024
+//   5.2 / 5.6, 2500 x 1024 6.0 / 6.0).
+// * Up to 2048 columns a CU has two.  Blocks whose columns straddle lines lose
+//   still (4096 x 1500 15.3 / 12.1, 8192 x 2000 25.3 / 24.3), aligned ones win
+//   until their few CUs are the bound (4096 x 2048 9.2 / 11.8, 8192 x 2048
+//   22.6 / 24.4, 16384 x 1536 42.6 / 42.1, 60000 x 2048 263 / 241).
+// * Beyond, the strips' partial lines are the bound (4096 x 8192 22.5 / 40.4,
+//   60000 x 4096 266 / 522, 8192 x 2200 26.3 / 31.7).
+// * With 4-byte loads the strips win where the rows' alignment varies and there
+//   are enough of them (4096 x 1001 15.6 / 9.2, 8192 x 333 25.5 / 12.9, 4096 x 10
+//   7.6 / 6.2, but 2049 x 333 5.1 / 5.9, 60000 x 1501 251 / 255), and lose where
+//   it does not (4096 x 512 one float off 7.8 / 10.2, 60000 x 1024 211 / 273).
+inline bool tall_strips(const float* x, int64_t rows, int64_t cols) {
+    if (rows <= 2048 || cols > 2048) return false;
+    if (!vec_rows(x, cols)) {
+        return cols % 8 != 0 && cols <= 1024 && (cols <= 128 || rows >= 3000);
+    }
+    if (cols <= 768) return true;
+    const bool whole_lines = cols % 32 == 0 && (reinterpret_cast<uintptr_t>(x) & 127u) == 0;
+    if (!whole_lines) return true;
+    return rows >= (cols <= 1024 ? 2500 : 16384);
+}
 
 template <bool VEC>
 __device__ __forceinline__ void colsum_tall_body(const float* __restrict__ x,
@@ -970,9 +1000,8 @@ hipError_t launch_relu_backward(const float* g, const float* act, float* out,
 hipError_t launch_colsum_sgd(const float* x, float* out, float* param, float lr,
                              int64_t rows, int64_t cols, hipStream_t stream) {
     if (cols == 0) return hipSuccess;
-    // (a launch holds at most 2^32 threads: wider matrices keep the 32-column blocks)
-    if (rows > kColsumShort && cols <= (int64_t(1) << 23)) {
-        const bool vec = cols % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+    if (tall_strips(x, rows, cols)) {
+        const bool vec = vec_rows(x, cols);
         const dim3 grid((unsigned)((cols + kTallCols - 1) / kTallCols));
         if (vec) {
             hipLaunchKernelGGL((colsum_tall_kernel<true>), grid, dim3(kTallThreads), 0, stream, x,
@@ -1080,9 +1109,6 @@ hipError_t launch_sgd_multi(int count, float* const* params,
 hipError_t launch_step_reduce(const float* G1, float* db1, int64_t hidden, const float* G2,
                               float* db2, int64_t classes, int64_t rows, const float* part,
                               int64_t nparts, int stride, float* loss, hipStream_t stream) {
-    auto vec = [](const float* x, int64_t cols) {
-        return cols % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
-    };
     // Sums wider than the strips are good for go to launch_colsum (a launch also
     // holds at most 2^32 threads, 2^24 columns in strips).
     constexpr int64_t kMaxCols = 2048;
@@ -1101,11 +1127,11 @@ hipError_t launch_step_reduce(const float* G1, float* db1, int64_t hidden, const
     hipLaunchKernelGGL((step_reduce_kernel<V1, V2>), grid, dim3(kTallThreads), 0, stream, G1,   \
                        db1, (int)hidden, n1, G2, db2, (int)classes, n2, rows, part, (int)nparts, \
                        stride, loss)
-    if (vec(G1, hidden)) {
-        if (vec(G2, classes)) FDL_STEP_REDUCE(true, true);
+    if (vec_rows(G1, hidden)) {
+        if (vec_rows(G2, classes)) FDL_STEP_REDUCE(true, true);
         else FDL_STEP_REDUCE(true, false);
     } else {
-        if (vec(G2, classes)) FDL_STEP_REDUCE(false, true);
+        if (vec_rows(G2, classes)) FDL_STEP_REDUCE(false, true);
         else FDL_STEP_REDUCE(false, false);
     }
 #undef FDL_STEP_REDUCE

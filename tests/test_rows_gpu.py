@@ -108,6 +108,25 @@ def test_softmax_xent_rows(device, batch, classes, shift):
     assert np.all(np.abs(host(d) - ref / batch) <= grad_tol)
 
 
+# both sides of the lines between strips of 4 columns and blocks of 32
+@pytest.mark.parametrize("rows,cols", [(2048, 64), (2049, 64), (2499, 1024), (2500, 1024),
+                                       (2600, 769), (3000, 1001), (2999, 333), (2100, 2044),
+                                       (2100, 2048), (2100, 2049), (16384, 1056), (4000, 512)])
+@pytest.mark.parametrize("shift", [0, 1, 4])
+def test_colsum_forms(device, rows, cols, shift):
+    import torch
+
+    x = rng(rows + cols + 1).standard_normal((rows, cols)).astype(np.float32)
+    d = _offset(x, shift)
+    out = torch.full((cols + 1,), float("nan"), device="cuda")
+    say(f"colsum forms {rows}x{cols} shift={shift}")
+    capi.colsum(d.data_ptr(), out.data_ptr(), rows, cols, stream())
+    # the longer of the two forms' chains: one of eight row groups of a block
+    bound = (rows / 8 + 16) * EPS * np.abs(x).astype(np.float64).sum(0)
+    assert np.all(np.abs(host(out)[:cols] - x.astype(np.float64).sum(0)) <= bound)
+    assert np.isnan(host(out)[cols])
+
+
 @pytest.mark.parametrize("rows,cols", [(2049, 1), (2049, 3), (3000, 4), (2100, 34), (4096, 36),
                                        (5119, 100), (9000, 257), (30001, 8)])
 @pytest.mark.parametrize("shift", [0, 1])
