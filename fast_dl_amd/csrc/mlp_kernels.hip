@@ -201,11 +201,14 @@ __global__ void add_row_bias_kernel(float* __restrict__ out,
 
 // out[i] = op(a[i], b[i]) over n floats.  HBM-bound: 16 bytes per lane and
 // access where every operand is 16-byte aligned (`out` may be `a` or `b`), one
-// float per lane otherwise and for the last n % 4.  Outputs of kStreamBytes or
-// more leave through non-temporal stores, since no cache would hold them for
-// their reader.  15.4M floats: relu 36.8 -> 18.5 us (6.6 TB/s), relu_backward
-// 51.6 -> 32.1 us (5.7 TB/s); 65k floats 2.2 -> 2.0 us.  More than one access
-// per thread was no faster (2, 4 and 8: within 3%).
+// float per lane otherwise and for the last n % 4.  Outputs of kStreamBytes, the
+// Infinity Cache's size, or more leave through non-temporal stores (2^26 floats:
+// relu 91 -> 79 us, with a pass over its output 178 -> 173, with a product
+// that reads it 315 -> 321); of smaller ones a part is still there when the
+// reader comes (60000 x 256: relu and a pass over its output 38.4 us, 42.7
+// with non-temporal stores).  15.4M floats: relu 25.8 -> 19.3 us (6.4 TB/s),
+// relu_backward 36.3 -> 27.2 us (6.8 TB/s).  More than one access per thread
+// was no faster (2, 4 and 8: within 3%).
 struct OpRelu {
     static constexpr bool kTwo = false;
     float lr;
@@ -257,7 +260,7 @@ elementwise_kernel(const float* a, const float* b, float* out, int64_t n, Op op)
     }
 }
 
-constexpr int64_t kStreamBytes = int64_t(32) << 20;
+constexpr int64_t kStreamBytes = int64_t(256) << 20;
 
 template <class Op>
 hipError_t launch_elementwise(const float* a, const float* b, float* out, int64_t n, Op op,
