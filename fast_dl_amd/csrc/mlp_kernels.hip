@@ -268,7 +268,9 @@ hipError_t launch_elementwise(const float* a, const float* b, float* out, int64_
     if (n == 0) return hipSuccess;
     const bool vec = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) |
                        reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
-    const dim3 grid(grid_for(vec ? n / 4 + n % 4 : n));
+    // (4 bytes per lane: four accesses per thread; with one each 2^23 floats one
+    // float off took sgd 19.1 us against 17.3, relu 16.1 against 12.8)
+    const dim3 grid(vec ? grid_for(n / 4 + n % 4) : grid_for(n, 4));
     if (!vec) {
         hipLaunchKernelGGL((elementwise_kernel<Op, false, false>), grid, dim3(kBlock), 0, stream,
                            a, b, out, n, op);
