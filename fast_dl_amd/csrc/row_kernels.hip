@@ -145,10 +145,11 @@ struct RowRegs {
     }
 };
 
-// out[r, :] = exp(x - max) / sum(exp(x - max)).
+// out[r, :] = exp(x - max) / sum(exp(x - max)).  (Here and below outputs may
+// lie over the inputs of the same place, so neither is __restrict__.)
 template <class Row>
 __global__ void __launch_bounds__(kRowThreads)
-softmax_kernel(const float* __restrict__ in, float* __restrict__ out, int64_t rows, int cols) {
+softmax_kernel(const float* in, float* out, int64_t rows, int cols) {
     const int lane = threadIdx.x % Row::G;
     const int64_t r = blockIdx.x * (int64_t)(kRowThreads / Row::G) + threadIdx.x / Row::G;
     const int64_t rc = r < rows ? r : rows - 1;  // a group past the end repeats the last row
@@ -164,8 +165,8 @@ softmax_kernel(const float* __restrict__ in, float* __restrict__ out, int64_t ro
 // batch (0 where the label is no class), and with grad_row its gradient
 // (softmax(z) - onehot) / batch.
 template <class Row>
-__device__ __forceinline__ float xent_row(const float* __restrict__ z, int64_t label, int classes,
-                                          float inv_b, int lane, float* __restrict__ grad_row) {
+__device__ __forceinline__ float xent_row(const float* z, int64_t label, int classes,
+                                          float inv_b, int lane, float* grad_row) {
     const bool valid = label >= 0 && label < classes;
     Row t;
     t.load(z, classes, lane);
@@ -197,9 +198,8 @@ __device__ __forceinline__ float xent_row(const float* __restrict__ z, int64_t l
 // memory.
 template <class Row>
 __global__ void __launch_bounds__(Row::kOneBlock)
-xent_kernel(const float* __restrict__ logits, const int64_t* __restrict__ labels,
-            float* __restrict__ part, float* __restrict__ grad, int64_t batch, int classes,
-            int64_t reserved) {
+xent_kernel(const float* logits, const int64_t* __restrict__ labels, float* part, float* grad,
+            int64_t batch, int classes, int64_t reserved) {
     const int lane = threadIdx.x % Row::G;
     const int per_block = blockDim.x / Row::G;
     const float inv_b = 1.0f / (float)batch;
@@ -223,9 +223,8 @@ xent_kernel(const float* __restrict__ logits, const int64_t* __restrict__ labels
 // then the gradients of the `reserved` rows that they lie in.
 template <class Row>
 __global__ void __launch_bounds__(Row::kOneBlock)
-xent_finish_kernel(const float* __restrict__ logits, const int64_t* __restrict__ labels,
-                   float* __restrict__ loss, float* grad, int64_t batch, int classes, int nparts,
-                   int64_t reserved) {
+xent_finish_kernel(const float* logits, const int64_t* __restrict__ labels, float* loss,
+                   float* grad, int64_t batch, int classes, int nparts, int64_t reserved) {
     const float lsum = thread_partials<Row::kOneBlock>(grad, nparts);
     // (block_sum's barrier comes after every thread's loads of the partial sums)
     const float s = block_sum(lsum);
@@ -267,8 +266,7 @@ __device__ __forceinline__ void wide_max_sum(const float* z, int64_t cols, float
 }
 
 __global__ void __launch_bounds__(kOneBlockThreads)
-softmax_wide_kernel(const float* __restrict__ in, float* __restrict__ out, int64_t rows,
-                    int64_t cols) {
+softmax_wide_kernel(const float* in, float* out, int64_t rows, int64_t cols) {
     for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
         const float* x = in + r * cols;
         float mx, s;
@@ -279,9 +277,8 @@ softmax_wide_kernel(const float* __restrict__ in, float* __restrict__ out, int64
     }
 }
 
-__device__ __forceinline__ float xent_wide_row(const float* __restrict__ z, int64_t label,
-                                               int64_t classes, float inv_b,
-                                               float* __restrict__ grad_row) {
+__device__ __forceinline__ float xent_wide_row(const float* z, int64_t label, int64_t classes,
+                                               float inv_b, float* grad_row) {
     const bool valid = label >= 0 && label < classes;
     const float zl = z[valid ? label : 0];
     float mx, s;
@@ -299,9 +296,8 @@ __device__ __forceinline__ float xent_wide_row(const float* __restrict__ z, int6
 
 // As xent_kernel: part[block] = the loss shares of its rows, in row order.
 __global__ void __launch_bounds__(kOneBlockThreads)
-xent_wide_kernel(const float* __restrict__ logits, const int64_t* __restrict__ labels,
-                 float* __restrict__ part, float* __restrict__ grad, int64_t batch,
-                 int64_t classes, int64_t reserved) {
+xent_wide_kernel(const float* logits, const int64_t* __restrict__ labels, float* part,
+                 float* grad, int64_t batch, int64_t classes, int64_t reserved) {
     const float inv_b = 1.0f / (float)batch;
     float lsum = 0.0f;
     for (int64_t r = blockIdx.x; r < batch; r += gridDim.x) {
@@ -314,8 +310,8 @@ xent_wide_kernel(const float* __restrict__ logits, const int64_t* __restrict__ l
 // As xent_finish_kernel; the partial sums all lie in row 0 (the host keeps
 // their number below `classes`).
 __global__ void __launch_bounds__(kOneBlockThreads)
-xent_wide_finish_kernel(const float* __restrict__ logits, const int64_t* __restrict__ labels,
-                        float* __restrict__ loss, float* grad, int64_t batch, int64_t classes,
+xent_wide_finish_kernel(const float* logits, const int64_t* __restrict__ labels,
+                        float* loss, float* grad, int64_t batch, int64_t classes,
                         int nparts) {
     const float s = block_sum(thread_partials<kOneBlockThreads>(grad, nparts));
     if (threadIdx.x == 0) loss[0] = s;
