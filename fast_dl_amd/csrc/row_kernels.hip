@@ -204,15 +204,16 @@ xent_kernel(const float* logits, const int64_t* __restrict__ labels, float* part
     const int per_block = blockDim.x / Row::G;
     const float inv_b = 1.0f / (float)batch;
     float lsum = 0.0f;
+    int turn = 0;  // the group's lanes take its rows' shares in turn, for short sums
     for (int64_t r0 = blockIdx.x * (int64_t)per_block; r0 < batch;
-         r0 += (int64_t)gridDim.x * per_block) {
+         r0 += (int64_t)gridDim.x * per_block, turn = (turn + 1) % Row::G) {
         const int64_t r = r0 + threadIdx.x / Row::G;
         const bool live = r < batch;
         const int64_t rc = live ? r : batch - 1;
         float* g = grad && live && r >= reserved ? grad + rc * classes : nullptr;
         const float share =
             xent_row<Row>(logits + rc * classes, labels[rc], classes, inv_b, lane, g);
-        if (live && lane == 0) lsum += share;
+        if (live && lane == turn) lsum += share;
     }
     if (!part) return;
     const float s = block_sum(lsum);
@@ -300,9 +301,14 @@ xent_wide_kernel(const float* logits, const int64_t* __restrict__ labels, float*
                  float* grad, int64_t batch, int64_t classes, int64_t reserved) {
     const float inv_b = 1.0f / (float)batch;
     float lsum = 0.0f;
+    float lost = 0.0f;  // what the additions to lsum rounded away (Kahan's summation)
     for (int64_t r = blockIdx.x; r < batch; r += gridDim.x) {
-        lsum += xent_wide_row(logits + r * classes, labels[r], classes, inv_b,
-                              grad && r >= reserved ? grad + r * classes : nullptr);
+        const float share = xent_wide_row(logits + r * classes, labels[r], classes, inv_b,
+                                          grad && r >= reserved ? grad + r * classes : nullptr);
+        const float y = share - lost;
+        const float t = lsum + y;
+        lost = fabsf(t) < INFINITY ? (t - lsum) - y : 0.0f;
+        lsum = t;
     }
     if (part && threadIdx.x == 0) part[blockIdx.x] = lsum;
 }

@@ -23,7 +23,7 @@ SHAPES = [(1, 1), (700, 1), (257, 4), (769, 4), (3, 5), (600, 16), (129, 17), (3
           (33, 65), (20, 68), (40, 128), (41, 129), (5, 256), (35, 257), (64, 260), (37, 512),
           (36, 513), (4, 1000), (2100, 1000), (50, 1023), (51, 1024), (34, 1025), (33, 1028),
           (7, 2047), (70, 2048), (2, 2049), (40, 2049), (3, 7000), (4500, 10),
-          (17000, 66), (70000, 3)]
+          (17000, 66), (70000, 3), (4100, 2051)]
 
 
 def _softmax64(z):
@@ -35,6 +35,29 @@ def _softmax64(z):
     bound = (8.0 + spread + np.sum(e * spread, 1, keepdims=True) / s
              + np.minimum(z.shape[1], 64)) * EPS
     return e / s, np.log(s[:, 0]) + m[:, 0], bound
+
+
+def loss_bound(z, lab):
+    """Each row's share of the loss times the batch, and a bound on the mean's error."""
+    batch, classes = z.shape
+    z64 = z.astype(np.float64)
+    m = z64.max(1)
+    e = np.exp(z64 - m[:, None])
+    s = e.sum(1)
+    lse = np.log(s) + m
+    at = np.flatnonzero((lab >= 0) & (lab < classes))
+    shares = np.zeros(batch)
+    shares[at] = lse[at] - z64[at, lab[at]]
+    # a share: log(sum) off by the sum's relative error (exponentials within 2 ulp, their
+    # arguments' rounding, its additions) and its own few roundings
+    spread = np.minimum(m[:, None] - z64, 200.0)
+    rel = 4.0 + np.sum(e * spread, 1) / s + min(classes, 64)
+    size = np.abs(lse) + np.abs(z64).max(1) + 1.0
+    # the mean: shares of one sign through at most `adds` additions (a lane's rows, the
+    # exchanges and the waves of a block, the partial sums of up to 4096 blocks)
+    adds = 60 + batch / 1024
+    tol = np.sum((rel + 4.0 * size)[at]) + adds * np.abs(shares).sum()
+    return shares, float(tol) * EPS / batch + 1e-30
 
 
 def _offset(a, shift):
@@ -80,15 +103,8 @@ def test_softmax_xent_rows(device, batch, classes, shift):
     capi.softmax_xent(d.data_ptr(), dl.data_ptr(), loss.data_ptr(), grad.data_ptr(), batch,
                       classes, stream())
     p, lse, bound = _softmax64(z)
-    valid = (lab >= 0) & (lab < classes)
-    at = np.flatnonzero(valid)
-    shares = np.zeros(batch)
-    shares[at] = lse[at] - z[at, lab[at]]
-    size = np.abs(lse) + np.abs(z).max(1) + 1.0
-    # each share rounds a few times, and passes through at most `adds` additions (a row
-    # group of one block takes every 16th row of wide ones)
-    adds = 160 + batch / 16
-    loss_tol = float(np.sum(size[at] * (bound.max(1)[at] + adds * EPS))) / batch + 1e-30
+    shares, loss_tol = loss_bound(z, lab)
+    at = np.flatnonzero((lab >= 0) & (lab < classes))
     ref = p.copy()
     ref[at, lab[at]] -= 1.0
     grad_tol = (bound * p + 3 * EPS * np.abs(ref)) / batch + 1e-37
@@ -106,6 +122,23 @@ def test_softmax_xent_rows(device, batch, classes, shift):
                       stream())
     assert abs(float(host(only)[0]) - shares.sum() / batch) <= loss_tol
     assert np.all(np.abs(host(d) - ref / batch) <= grad_tol)
+
+
+def test_loss_keeps_infinities(device):
+    # a row whose label is masked out loses without bound; the others' losses do not hide it
+    import torch
+
+    for batch, classes in ((40, 10), (300, 2050), (5000, 100)):
+        z = rng(classes).standard_normal((batch, classes)).astype(np.float32)
+        lab = np.zeros(batch, np.int64)
+        z[batch // 2, 0] = -np.inf
+        d, dl, loss = dev(z), dev(lab), torch.zeros(1, device="cuda")
+        say(f"loss infinity {batch}x{classes}")
+        for grad in (None, torch.empty_like(d)):
+            capi.softmax_xent(d.data_ptr(), dl.data_ptr(), loss.data_ptr(),
+                              grad.data_ptr() if grad is not None else None, batch, classes,
+                              stream())
+            assert float(host(loss)[0]) == np.inf
 
 
 # both sides of the lines between strips of 4 columns and blocks of 32
