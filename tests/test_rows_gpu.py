@@ -23,7 +23,7 @@ SHAPES = [(1, 1), (700, 1), (257, 4), (769, 4), (3, 5), (600, 16), (129, 17), (3
           (33, 65), (20, 68), (40, 128), (41, 129), (5, 256), (35, 257), (64, 260), (37, 512),
           (36, 513), (4, 1000), (2100, 1000), (50, 1023), (51, 1024), (34, 1025), (33, 1028),
           (7, 2047), (70, 2048), (2, 2049), (40, 2049), (3, 7000), (4500, 10),
-          (17000, 66), (70000, 3), (4100, 2051)]
+          (17000, 66), (70000, 3), (3073, 1), (4100, 2051)]
 
 
 def _softmax64(z):
