@@ -249,7 +249,10 @@ xent_finish_kernel(const float* logits, const int64_t* __restrict__ labels, floa
 
 // Rows too long for registers: a block of 1024 threads per row, which passes
 // over the row three times (maximum, sum, output); the later passes find it
-// in the L2.
+// in the L2.  Softmax takes 256 threads per row where there are rows enough to
+// fill the CUs with such blocks: 8192 x 2049 65.5 us with 1024, 41.5 with 256
+// (46.7 with a wave per row), 20000 x 4096 317 and 275; fewer or longer rows
+// need the more threads (2000 x 32000 205 and 218, 256 x 8192 9.4 and 17).
 __device__ __forceinline__ float wide_reduce(float x, bool is_max) {
     __shared__ float wred[kOneBlockThreads / kWaveLanes];
     x = is_max ? group_max<kWaveLanes>(x) : group_sum<kWaveLanes>(x);
@@ -369,8 +372,9 @@ hipError_t launch_softmax(const float* in, float* out, int64_t rows, int64_t col
     if (rows == 0 || cols == 0) return hipSuccess;
     if (cols > kMaxRegCols) {
         const unsigned blocks = (unsigned)std::min<int64_t>(rows, 1 << 20);
-        hipLaunchKernelGGL(softmax_wide_kernel, dim3(blocks), dim3(kOneBlockThreads), 0, stream,
-                           in, out, rows, cols);
+        const int threads = rows >= 4096 && cols <= 16384 ? kRowThreads : kOneBlockThreads;
+        hipLaunchKernelGGL(softmax_wide_kernel, dim3(blocks), dim3(threads), 0, stream, in, out,
+                           rows, cols);
         return hipGetLastError();
     }
     return with_row_regs(cols, rows_vec4(in, out, cols), [&](auto row) {
