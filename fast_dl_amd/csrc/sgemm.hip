@@ -3230,19 +3230,61 @@ const char* kernel_name(GemmKernel k) {
 
 namespace {
 
-// Time of the split-K kernel with `tile`-wide tiles, in us: the blocks run in
-// rounds of one per CU, each bound by its own serial K (the lines of A and B a
-// CU takes in).  Measured (us, 16 / 32 wide): 128x1024x1024 7.3 / 11.0,
-// 2048x100x1024 13.4 / 11.4, 1024x100x2048 13.7 / 19.7, 32x4096x4096
-// 26.7 / 35.9, 64x64x4096 11.6 / 34.6, 512^3 7.9 / 6.9, 700^3 19.0 / 16.2;
-// B k-contiguous (NT): 256x784x256 5.6 / 4.5, 2048x100x1024 15.8 / 10.3.
-double splitk_us(int tile, const GemmParams& p, bool transB, int64_t batch) {
+// Whether operands of this shape have rows that no 16-byte load takes whole.
+bool odd_rows(const GemmParams& p, bool transA, bool transB) {
+    return p.K % 4 != 0 || (transA ? p.M : p.K) % 4 != 0 || (transB ? p.K : p.N) % 4 != 0;
+}
+
+int64_t splitk_tiles(int tile, const GemmParams& p, int64_t batch) {
+    return (int64_t)((p.M + tile - 1) / tile) * ((p.N + tile - 1) / tile) * batch;
+}
+
+// The split-K kernel's tiles for K of at least 128.  A tile's K is serial, so
+// the blocks run in rounds of one per CU.  32-wide tiles move half the data
+// per output, 16-wide ones take 0.35 to 0.45 of their time per round.  Measured
+// on 481 products, over which this rule costs 0.3% on the faster form (us, 16 /
+// 32 wide):
+// * Fewer than 128 32-wide tiles leave half the CUs idle: 16 wide (64x64x4096
+//   11.6 / 34.6, 496x176x7920 46.3 / 68.1, 47x1904x1264 TN 13.3 / 14.6).
+// * Two rounds of 16-wide tiles against one: 16 wide (466x264x3351 25.4 /
+//   34.4, 1424x66x1088 TN 10.6 / 13.9).
+// * Four or five against two: 16 wide (336x768x5188 61 / 89, 3104x80x1529 NT
+//   21.3 / 28.2; five 1280x240x1344 20.5 / 26.8), but neither five rounds nor
+//   4-byte loads with a long K (467x608x17440 NT 300 / 247, 440x578x21034 385 /
+//   350, 800x354x3338 NT 59 / 55), nor five rounds of many small problems (79
+//   of 97x21x325 TN 12.7 / 9.9).
+// * Otherwise 32 wide (60x4000x2240 NT 35.9 / 21.9, 1053x202x13921 TN 190 /
+//   124, 48x7648x2512 67 / 47).
+// * At most 48 rows share the lines of a row-major B between three blocks,
+//   which use half of each: 16 wide pays in two short rounds of 16-byte loads
+//   only (16x4768x2512 TN 21.5 / 26.3, but 13x5472x27877 265 / 234, 40x2391x4604
+//   55.9 / 44.0, 48x5093x1696 TN 41.5 / 33.7).
+bool splitk_16_wide(const GemmParams& p, bool transA, bool transB, int64_t batch) {
     constexpr int64_t kCUs = 256;
-    const int64_t tiles =
-        (int64_t)((p.M + tile - 1) / tile) * ((p.N + tile - 1) / tile) * batch;
+    const int64_t t16 = splitk_tiles(16, p, batch), t32 = splitk_tiles(32, p, batch);
+    const int64_t rounds16 = (t16 + kCUs - 1) / kCUs, rounds32 = (t32 + kCUs - 1) / kCUs;
+    if (t32 < 128 || rounds16 == 1) return true;
+    if (p.M <= 48 && !transB) return rounds16 == 2 && p.N % 4 == 0 && p.K < 8000;
+    if (rounds16 == 2) return true;
+    if (rounds32 != 2) return false;
+    if (p.K >= 2000) return rounds16 <= 4 && !odd_rows(p, transA, transB);
+    return rounds16 <= (batch == 1 ? 5 : 4);
+}
+
+// Time of the split-K kernel with `tile`-wide tiles for one problem, in us
+// (fitted to the same products, within 20% of nine in ten).
+double splitk_us(int tile, const GemmParams& p, bool transB) {
+    constexpr int64_t kCUs = 256;
+    const int64_t tiles = splitk_tiles(tile, p, 1);
     const double rounds = (double)((tiles + kCUs - 1) / kCUs);
-    return tile == 16 ? 1.5 + (transB ? 0.0037 : 0.0029) * p.K * rounds
-                      : 2.0 + 0.0087 * p.K * rounds;
+    const double load = std::min(1.0, (double)tiles / kCUs);
+    if (tile == 32) {
+        return 3.3 + (0.0078 + 0.0015 * load - (transB ? 0.0012 : 0.0)) * p.K * rounds;
+    }
+    const bool one_block = p.M <= 8 && transB;  // (rows read once, by a block each)
+    if (rounds == 1) return 2.5 + (0.0026 - (one_block ? 0.0005 : 0.0) + 0.0010 * load) * p.K;
+    const double few_rows = p.M <= 48 && !transB ? 1.3 : 1.0;
+    return 1.5 + (one_block ? 0.0028 : transB ? 0.0034 : 0.0035) * few_rows * p.K * rounds;
 }
 
 }  // namespace
@@ -3255,7 +3297,7 @@ GemmKernel choose_kernel(const GemmParams& p, bool transA, bool transB,
     const int64_t t64 = (int64_t)((p.M + 63) / 64) * ((p.N + 63) / 64) * batch;
     constexpr int64_t kCUs = 256;
     // Too few 64x64 tiles to occupy the GPU: split K over the waves of a
-    // block instead, on 16x16 or 32x32 output tiles by splitk_us (short K: 16x16
+    // block instead, on 16x16 or 32x32 output tiles by splitk_16_wide (short K: 16x16
     // when 32x32 ones would leave most CUs idle).  With K >= 256 the 64x64 direct-to-LDS tile wins from ~160
     // tiles (777^3: 21.9 vs 25.2 us; 1024^3: 22 vs 42 us).  Short K (64 to
     // 255) needs a full GPU of 64x64 tiles (the C4 batch of 64 128x128x64
@@ -3269,11 +3311,9 @@ GemmKernel choose_kernel(const GemmParams& p, bool transA, bool transB,
     const bool long_k = p.K >= 256;
     if (p.K < 64 || t64 < (long_k ? 160 : kCUs) ||
         (!long_k && t128 < 128 && rem > 0 && rem < 64)) {
-        const int64_t t32 = (int64_t)((p.M + 31) / 32) * ((p.N + 31) / 32) * batch;
-        if (p.K < 128) return t32 < 128 ? GemmKernel::SplitK16 : GemmKernel::SplitK32;
-        return splitk_us(16, p, transB, batch) < splitk_us(32, p, transB, batch)
-                   ? GemmKernel::SplitK16
-                   : GemmKernel::SplitK32;
+        const bool wide16 = p.K < 128 ? splitk_tiles(32, p, batch) < 128
+                                      : splitk_16_wide(p, transA, transB, batch);
+        return wide16 ? GemmKernel::SplitK16 : GemmKernel::SplitK32;
     }
     // The direct-to-LDS tiles compete where their shape contract holds (the
     // 4-byte-copy ones almost always); the register-staged tiles only when
@@ -3374,10 +3414,9 @@ SlicePlan slice_plan(const GemmParams& p, bool transA, bool transB, int64_t batc
     if (direct != GemmKernel::SplitK16 && direct != GemmKernel::SplitK32) return s;
     // (operands that cannot take 16-byte loads cost the split-K kernels about a
     // fifth more than splitk_us says: 16x1001x4097 18.2 us, 32x3001x2003 15.7)
-    const bool odd = p.K % 4 != 0 || (transA ? p.M : p.K) % 4 != 0 ||
-                     (transB ? p.K : p.N) % 4 != 0;
+    const bool odd = odd_rows(p, transA, transB);
     const double direct_us = (odd ? 1.2 : 1.0) *
-        splitk_us(direct == GemmKernel::SplitK16 ? 16 : 32, p, transB, batch);
+        splitk_us(direct == GemmKernel::SplitK16 ? 16 : 32, p, transB);
     const int bm = p.M <= 32 ? 32 : 64, bn = 64;
     const int64_t tiles_m = (p.M + bm - 1) / bm, tiles_n = (p.N + bn - 1) / bn;
     const int64_t tiles = tiles_m * tiles_n;
