@@ -3396,48 +3396,49 @@ SkinnySplit skinny_split_plan(const GemmParams& p, bool transA, bool transB, int
 }
 
 // When and how a product runs as K slices.  Only where a split-K kernel would
-// run it (its tiles cannot fill the GPU): the slices' tiles in r rounds of one
-// per CU take about 8.4 us (two launches, the first tile's arrival, the sums'
-// round trip) plus 0.0150 us per step of K (64x64 tile; 0.0082 for 32x64), 2
-// us per further round and the partial sums' bytes.  Measured against the
-// split-K kernel (us): 32x4096x4096 17.5 / 26.4, 64x4096x4096 23.8 / 36.8,
-// 512x512x4096 24.4 / 36.7, 300x300x3000 14.0 / 21.1, 776x500x2000 23.9 /
-// 37.3, 784x256x60000 TN 214 / 515, odd 32x4097x4099 22.3 / 73.4 and
-// 777x250x5000 TN 28 / 47.6; where it predicts less than a tenth to gain the
-// single launch stays (256x256x1024 9 / 4.4, 16x4096x4096 17.8 / 16.7).  From
-// the shape alone, since the workspace query has no leading dimensions or
-// pointers: these choose between 16- and 4-byte copies of the same tile.
+// run it (its tiles cannot fill the GPU): the slices' tiles in rounds of one
+// per CU take about 7.2 us (two launches, the first tile's arrival) plus 0.0169
+// us per step of K (64x64 tile; 0.0104 for 32x64), 0.7 us per further round,
+// 0.08 us per slice in the sum (each of its threads reads them in turn) and the
+// partial sums' bytes, written and read; fitted to 407 plans, within 10% of
+// the time of nine in ten.  The single launch stays where the two are even: a
+// plan without the slices' own term takes 18 of them for 208x32x2231 TT, 11.9
+// us against 8.1, and 24 for 192x16x3190 TT, 12.5 against 10.7.
+// Measured, slices against one launch (us): 32x4096x4096 19.1 / 37.0,
+// 64x4096x4096 25.2 / 37.3, 512x512x4096 26.1 / 38.1, 777x250x5000 TN 30.0 /
+// 47.9, 784x256x60000 TN 224 / 522, 30x64x35509 25 / 89.  From the shape
+// alone, since the workspace query has no leading dimensions or pointers: these
+// choose between 16- and 4-byte copies of the same tile.
 SlicePlan slice_plan(const GemmParams& p, bool transA, bool transB, int64_t batch) {
     SlicePlan s;
     if (batch != 1 || p.M < 1 || p.N < 1 || p.K < 256) return s;
     const GemmKernel direct = choose_kernel(p, transA, transB, batch);
     if (direct != GemmKernel::SplitK16 && direct != GemmKernel::SplitK32) return s;
-    // (operands that cannot take 16-byte loads cost the split-K kernels about a
-    // fifth more than splitk_us says: 16x1001x4097 18.2 us, 32x3001x2003 15.7)
-    const bool odd = odd_rows(p, transA, transB);
-    const double direct_us = (odd ? 1.2 : 1.0) *
-        splitk_us(direct == GemmKernel::SplitK16 ? 16 : 32, p, transB);
     const int bm = p.M <= 32 ? 32 : 64, bn = 64;
     const int64_t tiles_m = (p.M + bm - 1) / bm, tiles_n = (p.N + bn - 1) / bn;
     const int64_t tiles = tiles_m * tiles_n;
     const double matrix = (double)slice_matrix(p.M, p.N) * sizeof(float);
-    const double per_step = bm == 32 ? 0.0082 : 0.0150;
+    const double per_step = bm == 32 ? 0.0104 : 0.0169;
     constexpr int64_t kCUs = 256;
     constexpr int kStep = 64;  // slices are whole K-tiles
     constexpr double kMaxBytes = 32 << 20;
-    double best_us = 0.9 * direct_us;
-    for (int rounds = 1; rounds <= 6; ++rounds) {
-        int64_t slices = rounds * kCUs / tiles;
+    const int64_t most = (int64_t)(kMaxBytes / matrix);
+    double best_us = 0.95 * splitk_us(direct == GemmKernel::SplitK16 ? 16 : 32, p, transB);
+    // Whole rounds of the CUs, and half and a quarter of one.  (Of the 32-row
+    // tiles a CU holds two: an odd round of a long K leaves it half empty,
+    // 1x2832x46962 NT 97 us in two rounds, 123 in three.)
+    for (const double rounds : {0.25, 0.5, 1.0, 2.0, 3.0, 4.0, 5.0, 6.0}) {
+        if (bm == 32 && (rounds == 3.0 || rounds == 5.0)) continue;
+        int64_t slices = std::min<int64_t>((int64_t)(rounds * kCUs / tiles), most);
         if (slices < 2) continue;
-        slices = std::min<int64_t>(slices, (int64_t)(kMaxBytes / matrix));
-        if (slices < 2) break;
         const int64_t steps =
             std::max<int64_t>(2 * kStep, ((p.K + slices - 1) / slices + kStep - 1) / kStep * kStep);
         slices = (p.K + steps - 1) / steps;
-        if (slices < 2) break;
+        if (slices < 2) continue;
         const int64_t run = (slices * tiles + kCUs - 1) / kCUs;
-        const double us = 8.4 + per_step * steps * run + 2.0 * (run - 1) +
-                          slices * matrix * 2.0 / 5.0e6;
+        const double us =
+            7.2 + per_step * steps * run + 0.7 * (run - 1) + 0.0825 * slices +
+            slices * matrix * 2.0 * 0.384e-6;
         if (us < best_us) {
             best_us = us;
             s.slices = (int)slices;

@@ -1,4 +1,4 @@
-"""Which split-K tiles a shape gets (no GPU).
+"""Which split-K tiles and which K slices a shape gets (no GPU).
 
 Shapes measured on both sides of the rules' lines: a product must not go to a
 form that takes longer than the one it would otherwise run on.
@@ -26,3 +26,26 @@ SPLITK16, SPLITK32 = capi.KERNEL_SPLITK16, capi.KERNEL_SPLITK32
 ])
 def test_splitk_tiles(ta, tb, M, N, K, batch, want):
     assert capi.kernel_choice(ta, tb, M, N, K, batch) == want
+
+
+@pytest.mark.parametrize("ta,tb,M,N,K", [
+    (1, 1, 208, 32, 2231),   # 8.1 us in one launch, 11.9 in slices
+    (1, 1, 560, 48, 3104),   # 11.4, 13.7
+    (1, 1, 192, 16, 3190),   # 10.7, 12.5
+    (1, 0, 33, 377, 3312),   # 12.0, 13.5
+    (0, 1, 32, 381, 2385),   # 9.2, 10.8
+    (1, 1, 80, 38, 2711),    # 9.6, 11.8
+])
+def test_no_slices_where_one_launch_is_faster(ta, tb, M, N, K):
+    assert capi.workspace_size(ta, tb, M, N, K) == 0
+
+
+@pytest.mark.parametrize("ta,tb,M,N,K", [
+    (0, 0, 32, 4096, 4096),    # 17.5 us in slices, 36.9 in one launch
+    (0, 0, 512, 512, 4096),    # 26, 38
+    (1, 0, 784, 256, 60000),   # 224, 524
+    (1, 0, 256, 256, 60000),   # 68, 172
+    (0, 0, 30, 64, 35509),     # 25, 89
+])
+def test_slices_where_they_are_faster(ta, tb, M, N, K):
+    assert 0 < capi.workspace_size(ta, tb, M, N, K) <= 32 << 20
