@@ -3253,6 +3253,9 @@ int64_t splitk_tiles(int tile, const GemmParams& p, int64_t batch) {
 //   4-byte loads with a long K (467x608x17440 NT 300 / 247, 440x578x21034 385 /
 //   350, 800x354x3338 NT 59 / 55), nor five rounds of many small problems (79
 //   of 97x21x325 TN 12.7 / 9.9).
+// * At most three times the rounds, with a K so short that a launch's fixed time
+//   counts, and rows enough to share B's lines: 16 wide (464x288x608 7.9 / 8.6,
+//   215x2432x564 17.9 / 20.6, 1328x136x323 5.4 / 5.6).
 // * Otherwise 32 wide (60x4000x2240 NT 35.9 / 21.9, 1053x202x13921 TN 190 /
 //   124, 48x7648x2512 67 / 47).
 // * At most 48 rows share the lines of a row-major B between three blocks,
@@ -3266,6 +3269,7 @@ bool splitk_16_wide(const GemmParams& p, bool transA, bool transB, int64_t batch
     if (t32 < 128 || rounds16 == 1) return true;
     if (p.M <= 48 && !transB) return rounds16 == 2 && p.N % 4 == 0 && p.K < 8000;
     if (rounds16 == 2) return true;
+    if (p.K < 850 && p.M >= 160 && !transB && rounds16 <= 3 * rounds32) return true;
     if (rounds32 != 2) return false;
     if (p.K >= 2000) return rounds16 <= 4 && !odd_rows(p, transA, transB);
     return rounds16 <= (batch == 1 ? 5 : 4);

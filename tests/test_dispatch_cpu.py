@@ -22,6 +22,8 @@ SPLITK16, SPLITK32 = capi.KERNEL_SPLITK16, capi.KERNEL_SPLITK32
     (0, 0, 336, 768, 5188, 1, SPLITK16),     # 61, 89
     (0, 0, 496, 176, 7920, 1, SPLITK16),     # 46.3, 68.1
     (0, 0, 32, 2293, 848, 1, SPLITK16),      # 7.9, 11.2
+    (0, 0, 464, 288, 608, 1, SPLITK16),      # 7.9, 8.6
+    (0, 0, 512, 512, 512, 1, SPLITK32),      # 7.9, 6.9
     (1, 0, 16, 4768, 2512, 1, SPLITK16),     # 21.5, 26.3
 ])
 def test_splitk_tiles(ta, tb, M, N, K, batch, want):
