@@ -487,13 +487,25 @@ int fdl_mlp2_train_step(const float* X, const int64_t* labels, int64_t batch,
     // below, whose 32x32 tiles are for products too small for the GPU.  From
     // how many multiply-adds in the first layer, by what the grouped form's
     // head costs; measured (us, grouped / one launch per product): three
-    // launches 2048x784x256x10 61 / 72, 3000x1000x256x10 104 / 84,
-    // 4096x1024x256x32 158 / 97; four 600x784x700x10 66 / 81,
-    // 4096x400x300x12 130 / 97; six 512x784x512x100 57 / 61, 1024x200x700x20
-    // 81 / 59, 2048x784x1024x100 243 / 159, 3520x364x912x18 312 / 162.
+    // launches 2048x784x256x10 67 / 77, 3000x1000x256x10 107 / 87,
+    // 4096x1024x256x32 159 / 99; four 600x784x700x10 69 / 85,
+    // 4096x400x300x12 133 / 101; six 1024x200x700x20 85 / 64,
+    // 2048x784x1024x100 246 / 163, 3520x364x912x18 315 / 167.  Short batches into
+    // narrow layers near the last line take up to 15% longer in slices, at
+    // three quarters of the error (512x784x512x100 60 / 64, dW1 1.4e-7 / 1.0e-7
+    // of its norm; 256x1024x512x64 44 / 50).
+    // Without dX three launches are two thirds of the work and dW1 has no
+    // scratch to be sliced in: they win until its own tiles fill the GPU
+    // (2048x784x256x10 42 / 62, 60000x784x256x10 606 / 1038, 4087x537x901x4
+    // 169 / 177, against 4096x784x1024x10 213 / 169, 4080x680x927x13 196 /
+    // 167), with dW1's error that of their longer sums (3000x1000x256x10 2.0e-7
+    // of its norm, 60000x784x256x10 8.5e-7; one launch each 0.9e-7 and 2.2e-7).
     // (dW1 has to hold the loss's partial sums.)
     const double size = (double)B * (double)I * (double)Hd;
-    if (size >= (three ? 6.0e8 : fused_head ? 4.0e8 : 1.2e8) && I * Hd >= fdl::xent_parts(B, Cc)) {
+    const int64_t dw1_tiles = ((I + 63) / 64) * ((Hd + 63) / 64);
+    const bool large = three ? (dX ? size >= 6.0e8 : size >= 1.5e9 && dw1_tiles >= 160)
+                             : size >= (fused_head ? 4.0e8 : 1.2e8);
+    if (large && I * Hd >= fdl::xent_parts(B, Cc)) {
         return large_step_backward(X, labels, B, I, Hd, Cc, W1, b1, W2, b2, lr, H, logits, G2, G1,
                                    dW1, db1, dW2, db2, dX, loss, hs);
     }

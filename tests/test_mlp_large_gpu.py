@@ -84,6 +84,22 @@ def test_large_step_repeats_bit_for_bit(device):
     assert all(np.array_equal(a[k], b[k]) for k in a)
 
 
+def test_large_step_without_dx(device):
+    # without dX the step takes one launch per product only where dW1's tiles fill the GPU
+    g = rng(8)
+    B, I, Hd, C = 2300, 820, 810, 10
+    X = g.random((B, I)).astype(np.float32)
+    labels = g.integers(0, C, B).astype(np.int64)
+    params = [(g.standard_normal(s) * k).astype(np.float32)
+              for s, k in (((I, Hd), np.sqrt(2.0 / I)), (Hd, 0.1), ((Hd, C), np.sqrt(2.0 / Hd)),
+                           (C, 0.1))]
+    say(f"large step without dX B={B} I={I} H={Hd} C={C}")
+    gpu = _step(X, labels, params, None)
+    ex = exact_step(X, labels, *params, LR)
+    ratios = worst_ratio(gpu, ex, step_bounds(X, labels, *params, LR, ex))
+    assert max(ratios.values()) <= 1.0, ratios
+
+
 @pytest.mark.parametrize("B,I,Hd,C", [(2, 4, (1 << 24) + 8, 3), (130, 260, 4100, 40),
                                       (64, 800, 2500, 2052)])
 def test_large_step_wide_layers(device, B, I, Hd, C):
