@@ -199,9 +199,12 @@ int large_step_backward(const float* X, const int64_t* labels, int64_t B, int64_
         p.epilogue = epi;
         return p;
     };
-    const bool aligned = (reinterpret_cast<uintptr_t>(dX) & 15u) == 0;
-    float* scratch = aligned ? dX : nullptr;
-    const size_t scratch_bytes = scratch ? (size_t)(B * I) * sizeof(float) : 0;
+    // From dX's first 16-byte boundary on, unless that skips some of it and the
+    // batch is short: then one launch per product is as fast (1385x213x552x17
+    // one float off 65 us against 75; 60000x784x256x10 1303 against 840).
+    const int64_t skip = (int64_t)(-reinterpret_cast<uintptr_t>(dX) % 16 / sizeof(float));
+    float* scratch = dX && (skip == 0 || (B >= 2048 && skip < B * I)) ? dX + skip : nullptr;
+    const size_t scratch_bytes = scratch ? (size_t)(B * I - skip) * sizeof(float) : 0;
     int st;
     // logits, G2 = dL/dlogits, G1 = (G2 W2^T) * [H > 0] and the loss's partial sums
     int64_t nparts = fdl::head_blocks(B);
