@@ -3615,7 +3615,7 @@ hipError_t launch_weight_grad(const GemmParams& p, bool transA, bool transB, flo
         SlicePlan s;
         const int64_t steps = ((p.K + slices - 1) / slices + kStep - 1) / kStep * kStep;
         s.kslice = (int)std::max<int64_t>(2 * kStep, steps);
-        s.slices = (p.K + s.kslice - 1) / s.kslice;
+        s.slices = (int)(((int64_t)p.K + s.kslice - 1) / s.kslice);
         const hipError_t err = s.slices >= 2
                                    ? launch_slice_plan(p, transA, transB, s, scratch, stream)
                                    : hipErrorInvalidValue;
