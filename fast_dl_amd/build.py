@@ -6,7 +6,7 @@ Compiles, in-tree, with hipcc for gfx950 only:
   ``include/fastdl_gemm.h`` and ``include/fastdl_data.h``;
 * ``fast_dl_amd/libfastdl.so`` -- the C++ ``dl::`` tensor/ops/nn API
   (``include/dl``) hosted on the HIP runtime, linked against the former;
-* ``fast_dl_amd/_fastcall.so`` -- the CPython side of ``fast_dl_amd.capi``'s calls;
+* ``fast_dl_amd/_fastcall<ABI tag>.so`` -- the CPython side of ``fast_dl_amd.capi``'s calls;
 * the C++ API test programs under ``tests/cpp`` (``tests/cpp/bin``).
 
 Every call rebuilds everything (the driver uses this as the "does it build"
@@ -116,7 +116,8 @@ def build_dl_library() -> str | None:
 
 def build_python_module() -> str:
     src = os.path.join(CSRC, "python", "fastcall.cpp")
-    out = os.path.join(PKG, "_fastcall.so")
+    # The ABI tag keeps another Python version from loading it (capi then calls through ctypes).
+    out = os.path.join(PKG, "_fastcall" + sysconfig.get_config_var("EXT_SUFFIX"))
     tmp = out + ".tmp"
     _run([HOST_CXX, "-O2", "-fPIC", "-std=c++17", "-Wall", "-shared", "-I", INCLUDE,
           "-I", sysconfig.get_paths()["include"], src, "-o", tmp])

@@ -7,14 +7,16 @@ import ctypes
 import os
 import subprocess
 import sys
+import sysconfig
 
 import numpy as np
 import pytest
 
 import fast_dl_amd.capi as capi
+# (built with the library: one that is missing or does not load is a failure)
+from fast_dl_amd import _fastcall as fastcall
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-fastcall = pytest.importorskip("fast_dl_amd._fastcall")
 
 EMPTY_GEMM = (0, 0, 0, 4, 4, None, 4, 0, None, 4, 0, None, 4, 0, 1, None, None, 0)
 # calls of every argument kind: ints, pointers as int and None, floats, sizes
@@ -76,3 +78,8 @@ def test_library_loads_on_the_first_call():
             "assert c.relu(None, None, 0, 0) == 0 and c._LIB is not None\n"
             "assert c.relu(None, None, 0, 0) == 0\n")
     subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True, timeout=120)
+
+
+def test_module_carries_this_pythons_abi_tag():
+    assert os.path.basename(fastcall.__file__) == \
+        "_fastcall" + sysconfig.get_config_var("EXT_SUFFIX")
