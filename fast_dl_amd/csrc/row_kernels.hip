@@ -52,18 +52,17 @@ __device__ __forceinline__ float group_sum(float x) {
     return x;
 }
 
-// Sum over a block (a multiple of 64 threads), on thread 0: each wave's lanes
-// by a fixed exchange tree, then the waves in order.
+// Sum over a block (a multiple of 64 threads, at most 1024), on thread 0: each
+// wave's lanes by a fixed exchange tree, then the waves' sums by another (one
+// after the other, their additions doubled the error of a small batch's loss).
 __device__ __forceinline__ float block_sum(float x) {
     __shared__ float wsum[kOneBlockThreads / kWaveLanes];
     x = group_sum<kWaveLanes>(x);
     if ((threadIdx.x & (kWaveLanes - 1)) == 0) wsum[threadIdx.x / kWaveLanes] = x;
     __syncthreads();
-    float s = 0.0f;
-    if (threadIdx.x == 0) {
-        for (unsigned w = 0; w < blockDim.x / kWaveLanes; ++w) s += wsum[w];
-    }
-    return s;
+    constexpr int kWaves = kOneBlockThreads / kWaveLanes;
+    static_assert(kWaves == 16, "one exchange group of 16 lanes");
+    return group_sum<kWaves>(threadIdx.x < blockDim.x / kWaveLanes ? wsum[threadIdx.x] : 0.0f);
 }
 
 // Thread t's share of `nparts` <= kMaxRowBlocks partial sums, t, t + NT, ...

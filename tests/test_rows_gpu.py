@@ -124,6 +124,34 @@ def test_softmax_xent_rows(device, batch, classes, shift):
     assert np.all(np.abs(host(d) - ref / batch) <= grad_tol)
 
 
+@pytest.mark.parametrize("batch,classes", [(256, 10), (1000, 100), (8192, 1500), (300, 4000),
+                                           (5000, 2100)])
+def test_loss_error_is_that_of_short_sums(device, batch, classes):
+    """Over seeds, the loss is off by about its last place, with a gradient and without.
+
+    Shares and sums rounded independently leave about half a unit in the last place
+    (6e-8) of a sum of few levels; one long chain of additions shows as several.
+    """
+    import torch
+
+    err = {"both": [], "loss": []}
+    say(f"loss error {batch}x{classes}")
+    for seed in range(16):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        z = torch.randn(batch, classes, generator=g, device="cuda") * 2
+        y = torch.randint(0, classes, (batch,), generator=g, device="cuda")
+        at = torch.arange(batch, device="cuda")
+        want = float(-torch.log_softmax(z.double(), 1)[at, y].mean())
+        loss, grad = torch.empty(1, device="cuda"), torch.empty_like(z)
+        for form in err:
+            capi.softmax_xent(z.data_ptr(), y.data_ptr(), loss.data_ptr(),
+                              grad.data_ptr() if form == "both" else None, batch, classes,
+                              stream())
+            err[form].append((float(host(loss)[0]) - want) / want)
+    for form, e in err.items():
+        assert np.sqrt(np.mean(np.square(e))) <= 1.2e-7, form
+
+
 def test_loss_keeps_infinities(device):
     # a row whose label is masked out loses without bound; the others' losses do not hide it
     import torch
