@@ -228,8 +228,9 @@ int fdl_relu_backward(const float* grad_out, const float* act, float* grad_in,
                       int64_t n, void* stream);
 
 /*
- * out[c] = sum_r x[r, c] (rows summed in increasing r order).  The db term of
- * linear backward, legacy/src/ops/Layers.cpp:44.
+ * out[c] = sum_r x[r, c], the rows added in a fixed order (results repeat bit
+ * for bit; not the order of r).  The db term of linear backward,
+ * legacy/src/ops/Layers.cpp:44.
  */
 int fdl_colsum(const float* x, float* out, int64_t rows, int64_t cols,
                void* stream);
@@ -280,13 +281,17 @@ int fdl_sgd_update(float* param, const float* grad, float lr, int64_t n,
  *
  * Every buffer belongs to the caller; the step allocates nothing.  H, logits,
  * G2, G1, dW1, db1, dW2, db2 hold the step's intermediates on return.
- * The step is 4 launches when classes <= 16 and hidden <= 1024, or
- * classes <= 32 and hidden <= 512, and ceil(batch / 8) * (classes + 1) <=
- * in_features * hidden: then dW1 holds per-block partial sums of the loss
- * and db2 until the last launch writes the weight gradient into it.
- * Otherwise it is 6 launches.  Large layers take one launch per product, and
- * one for all updates; dX then holds partial sums of the weight gradients
- * until its own product writes it.
+ * With dX, hidden <= 256 and a multiple of 4, classes <= 32 and H and W1
+ * 16-byte aligned the step is 3 launches.  Else, when classes <= 16 and hidden
+ * <= 1024, or classes <= 32 and hidden <= 512, and ceil(batch / 8) *
+ * (classes + 1) <= in_features * hidden, it is 4, or 3 without dX.  Otherwise
+ * it is 6.  Large layers take a launch per product, one for all updates and a
+ * few for sums.
+ * dW1 and dX also serve as scratch, each until the launch that writes its own
+ * values: dW1 for partial sums of the loss and db2 in the forms of 4, and of 3
+ * without dX, and of the loss in the large form, dX for partial sums of the
+ * products in the large form.  Work on other streams must not read them while
+ * a step is in flight.
  */
 int fdl_mlp2_train_step(const float* X, const int64_t* labels,
                         int64_t batch, int64_t in_features,
