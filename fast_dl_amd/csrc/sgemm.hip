@@ -3242,7 +3242,7 @@ int64_t splitk_tiles(int tile, const GemmParams& p, int64_t batch) {
 // The split-K kernel's tiles for K of at least 128.  A tile's K is serial, so
 // the blocks run in rounds of one per CU.  32-wide tiles move half the data
 // per output, 16-wide ones take 0.35 to 0.45 of their time per round.  Measured
-// on 481 products, over which this rule costs 0.3% on the faster form (us, 16 /
+// on 590 products, over which this rule costs 0.5% on the faster form (us, 16 /
 // 32 wide):
 // * Fewer than 128 32-wide tiles leave half the CUs idle: 16 wide (64x64x4096
 //   11.6 / 34.6, 496x176x7920 46.3 / 68.1, 47x1904x1264 TN 13.3 / 14.6).
